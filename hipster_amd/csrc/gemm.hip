@@ -9,14 +9,11 @@
 //   qmm_gemm_bf16           hip::BlasLt::gemm     engine/kernels/gemm.hip:125-160 (own MFMA kernel, no hipBLASLt)
 //   qmm_f32_to_bf16, qmm_bf16_to_f32, qmm_bf16_to_f32_seg, qmm_bf16_to_f32_seg2   gemm.hip:77-95
 //
-// Q4_K GEMM (qmm_gemm_wq): 256 x 256 output tiles, K step 64, 512 threads (two waves per SIMD, so
-// one wave's MFMAs hide the other's dequantisation), v_mfma_f32_32x32x16_bf16.  A streams
-// global -> LDS by DMA three stages ahead; a K step of 64 is exactly one 32-byte qs "pair" of each
-// weight row's block, dequantised from registers into a two-stage bf16 W ring.  bf16 GEMM
-// (qmm_gemm_bf16): 256 x 256 tiles, 4 waves, v_mfma_f32_16x16x32_bf16, register-staged two-stage
-// LDS ring.  Both map workgroups XCD-aware: consecutive workgroup ids go to different XCDs, so tile
-// ids are assigned so that the M tiles of one weight tile run on the same XCD and share its L2.
+// qmm_gemm_wq and qmm_gemm_bf16 run the tile kernel of gemm_tile.hpp with the weight source as a template
+// argument; pick_tile below chooses its tile by the shape.  qmm_gemm_bf16_ld keeps a kernel without buffer
+// resources (256 x 256 tiles, register-staged two-stage LDS ring) for row strides that no resource spans.
 #include "fmt_dequant.hpp"
+#include "gemm_tile.hpp"
 #include "qmm_common.hpp"
 
 #include <hip/hip_runtime.h>
@@ -133,7 +130,7 @@ __global__ void k_bf16_to_f32_seg2(const uint16_t* __restrict__ x, const uint16_
 }
 
 // ------------------------------------------------------------------------------------------
-// bf16 x bf16 MFMA GEMM (the BlasLt::gemm twin).  Macro tile GBM x GBN = 256 x 256, K step 64, 4 waves as 2 x 2, each wave a
+// bf16 x bf16 MFMA GEMM for row strides beyond the tile kernel's buffer resources.  Macro tile GBM x GBN = 256 x 256, K step 64, 4 waves as 2 x 2, each wave a
 // 128 x 128 tile = 8 x 8 MFMA tiles of 16 x 16 (256 f32 accumulators per lane, held in AGPRs).
 // LDS holds two stages of {A 256 x 64, W 256 x 64} bf16 with rows padded to 72 elements (144 B):
 // the 16-byte fragment reads of 16 consecutive rows then fall on 16 distinct 4-bank groups.
@@ -262,265 +259,65 @@ __global__ void __launch_bounds__(256) k_gemm(const uint16_t* __restrict__ A, co
         }
     }
 }
-
 // ------------------------------------------------------------------------------------------
-// Fused Q4_K GEMM with DMA-staged A.  The A tile goes global -> LDS with global_load_lds_dwordx4 (no
-// registers), three stages deep; the bf16 W tile, dequantised from Q4_K registers, two stages.
-// Stage layout: 256 rows x 8 chunks of 16 B, unpadded, chunk c of row r stored in slot
-// r*8 + (c ^ ((r >> 1) & 7)): a DMA instruction writes 1 KiB of consecutive slots (lane i -> slot
-// base + i, so the swizzle is applied to the global address each lane fetches), and the 16
-// consecutive rows of an MFMA fragment read land on 16 distinct 4-bank groups.
-// Step s: DMA A tile s+2 -> A stage (s+2)%3; MFMAs of tile s (A stage s%3, W stage s%2); tile s+1's
-// W registers -> W stage (s+1)%2; W tile s+2 -> registers; wait; barrier.  The A tile thus has two
-// steps of MFMA time to land.
-constexpr int kChunks = GBM * GBK / 8;                         // 16-byte chunks per stage (2048)
+// Tile choice of the dequantising GEMM (gemm_tile.hpp).  A workgroup fills a CU, so a shape takes
+// ceil(tiles / CUs) rounds of ceil(K / 64 / KS) steps each, and the choice is the tile with the least
+// rounds x (steps x step time + launch and reduction).  Step times in 0.01 us, measured with Q4_K weights on
+// 256 CUs: large tiles do the most work per step (192 x 256: 34 blocks of 32 x 32 x 64 per us, 32 x 32 with
+// eight K groups: 9) and small ones fill the chip where M x N is small.  The choice does not look at the
+// format, so every weight source gets the same K order.
+struct TileShape { int nrb, cw, ks, step, fixed; };
+constexpr TileShape kTiles[] = {{1, 1, 8, 90, 400}, {2, 1, 8, 125, 500}, {2, 2, 4, 87, 500}, {4, 2, 4, 116, 600}, {4, 4, 2, 102, 600},
+                                {4, 8, 1, 98, 600}, {5, 8, 1, 122, 600}, {6, 8, 1, 139, 600}, {8, 8, 1, 156, 600}};
+constexpr int kNumTiles = (int)(sizeof(kTiles) / sizeof(kTiles[0]));
 
-// The five stages are separate LDS variables and every access names its stage at compile time (the
-// K loop is unrolled by 6 = 3 A stages x 2 W stages).  The compiler then knows which stage each DMA
-// writes, so an LDS read waits only for DMA into its own stage, and its count of the W register
-// loads stays exact (with one LDS array it would wait for every DMA in flight before each read).
-__shared__ uint4 gA0[kChunks], gA1[kChunks], gA2[kChunks], gB0[kChunks], gB1[kChunks];
-template <int S>
-__device__ __forceinline__ uint4* ga() {
-    if constexpr (S == 0) return gA0;
-    else if constexpr (S == 1) return gA1;
-    else return gA2;
-}
-template <int S>
-__device__ __forceinline__ uint4* gb() {
-    if constexpr (S == 0) return gB0;
-    else return gB1;
-}
-template <int V>
-using IC = std::integral_constant<int, V>;
-
-// Workgroup barrier for a kernel whose DMA into LDS is still in flight on purpose.  A workgroup
-// release fence on LDS would wait for every outstanding DMA (vmcnt(0)); here the release is at wave
-// scope (it only keeps the compiler from moving LDS accesses across it), this wave's own LDS stores
-// are retired with lgkmcnt(0), and the DMA a reader depends on has been waited for explicitly with
-// vmcnt(n) before the barrier.
-__device__ __forceinline__ void lds_barrier_dma() {
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-    __builtin_amdgcn_s_waitcnt(0xC07F);       // lgkmcnt(0)
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-    __builtin_amdgcn_sched_barrier(0);
+int tile_count(const TileShape& t, int M, int N) {
+    return ((M + 32 * t.nrb - 1) / (32 * t.nrb)) * ((N + 32 * t.cw - 1) / (32 * t.cw));
 }
 
-__device__ __forceinline__ int swz(int r, int c) { return r * 8 + (c ^ ((r >> 1) & 7)); }
-
-// 32 x 32 x 16 MFMA tiles.  Operand layout (v_mfma_f32_32x32x16_bf16): lane l supplies row (or
-// column) l%32 and the 8 consecutive k values 8*(l/32)..+7 of the 16-wide K slice; output element i
-// of lane l is row 8*(i/4) + 4*(l/32) + i%4, column l%32.  Fragment row R = base + 32*t + l%32 keeps
-// (R >> 1) & 7 == ((l%32) >> 1) & 7, so fragment t of slice ks sits at lane base + 256*t chunks.
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-// ------------------------------------------------------------------------------------------
-// Two waves per SIMD ("ping-pong"): 512 threads, 8 waves as 2 (M) x 4 (N), wave tile 128 x 64 =
-// 4 x 2 MFMA tiles of 32 x 32 (128 accumulators per lane).  The two waves of a SIMD interleave in
-// hardware: while one issues MFMAs the other runs its W dequantisation, DMA issue and fragment
-// reads, so the non-MFMA work of a step hides under the other wave's MFMAs.  Each W row is
-// dequantised by two threads, one sub-block (32 weights) each.
-constexpr int kPPThreads = 512;
-
-__device__ __forceinline__ void dma_a_pp(const uint16_t* __restrict__ A, int M, int lda, int m0, int k0, uint4* La) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        // chunk slot p = (4w + i) * 64 + lane: row r = 32w + 8i + lane/8, slot column lane%8
-        const int r = 32 * wave + 8 * i + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
-        const uint32_t off = (uint32_t)min(m0 + r, M - 1) * (uint32_t)lda + (uint32_t)(k0 + 8 * c);
-        __builtin_amdgcn_global_load_lds(A + off, La + (4 * wave + i) * 64, 16, 0, 0);
-    }
+// the operands' span in a tile must fit a buffer resource (32-bit offsets)
+bool tile_fits(const TileShape& t, const GemmArgs& a) {
+    const size_t ra = (size_t)std::min(a.M, 32 * t.nrb) - 1, rw = (size_t)std::min(a.N, 32 * t.cw) - 1;
+    return ra * a.lda + (size_t)a.K * 2 <= 0xffffffffu && rw * a.ldw + a.rowbytes <= 0xffffffffu;
 }
 
-struct WRawQ4KHalf {
-    uint4 hd, q0, q1;
-    __device__ __forceinline__ void load(const uint8_t* __restrict__ W, int N, int K, int, int n0, int k0) {
-        const int n = min(n0 + (int)(threadIdx.x >> 1), N - 1);
-        const uint8_t* bp = W + (size_t)n * ((size_t)(K >> 8) * 144) + (size_t)(k0 >> 8) * 144;
-        const int j = (k0 >> 6) & 3;
-        hd = ld16(bp);
-        q0 = ld16(bp + 16 + 32 * j);
-        q1 = ld16(bp + 32 + 32 * j);
+int pick_tile(const GemmArgs& a) {
+    int best = -1;
+    long long cost = 0;
+    const int cus = device_cu_count(), nk = a.K / 64;
+    for (int i = 0; i < kNumTiles; ++i) {
+        const TileShape& t = kTiles[i];
+        if (!tile_fits(t, a)) continue;
+        const long long rounds = (tile_count(t, a.M, a.N) + cus - 1) / cus;
+        const long long c = rounds * ((long long)((nk + t.ks - 1) / t.ks) * t.step + t.fixed);
+        if (best < 0 || c < cost) { best = i; cost = c; }
     }
-    // thread t: row t/2, sub-block 2j + (t&1): 32 bf16 -> chunks 4*(t&1)..+3 of the row, each weight
-    // bf16(fmaf(dl, q, -ml)) through v_fma_mix_f32 (q4_bf16x8_mix: the low nibbles with dl * 2^24, the
-    // high ones in place with dl * 2^20)
-    __device__ __forceinline__ void store(uint4* Lb, int k0) const {
-        const int t = threadIdx.x, h = t & 1, row = t >> 1;
-        const int sbi = 2 * ((k0 >> 6) & 3) + h;
-        const float d = h2f(hd.x), dmin = h2f(hd.x >> 16);
-        const Q4kScaleBytes sb = q4k_scale_bytes(hd.y, hd.z, hd.w);
-        const float dl = d * (float)byte8(sb.sc_lo, sb.sc_hi, sbi), ml = dmin * (float)byte8(sb.m_lo, sb.m_hi, sbi);
-        const float s24 = dl * (h ? 1048576.f : 16777216.f);
-        const uint32_t m = h ? 0x00f000f0u : 0x000f000fu;
-        const uint32_t qw[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const qmm_bf16x8 v = q4_bf16x8_mix(qw[2 * c], qw[2 * c + 1], m, s24, -ml);
-            Lb[swz(row, 4 * h + c)] = __builtin_bit_cast(uint4, v);
-        }
-    }
-};
-
-// W from bf16 rows [N][K] (the BlasLt::gemm twin): thread t copies the 32 weights of row t/2, half t&1
-// of the step, a step ahead
-struct WRawBf16Half {
-    SubRaw r;                               // r.v[0..3]: the 64 bytes
-    __device__ __forceinline__ void load(const uint8_t* __restrict__ W, int N, int, int ldw, int n0, int k0) {
-        const int n = min(n0 + (int)(threadIdx.x >> 1), N - 1);
-        const uint16_t* p = (const uint16_t*)W + (size_t)n * ldw + k0 + 32 * (threadIdx.x & 1);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) r.v[c] = ld16(p + 8 * c);
-    }
-    __device__ __forceinline__ void store(uint4* Lb, int) const {
-        const int t = threadIdx.x, h = t & 1, row = t >> 1;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) Lb[swz(row, 4 * h + c)] = r.v[c];
-    }
-};
-
-// W in one of the other quantised formats: thread t loads the raw bytes of row t/2's sub-block
-// (k0/32 + (t&1)) a step ahead and dequantises them exactly (as qmm_dequant_bf16), RNE to bf16
-template <int F>
-struct WRawFmtHalf {
-    SubRaw r;
-    __device__ __forceinline__ void load(const uint8_t* __restrict__ W, int N, int K, int, int n0, int k0) {
-        const int n = min(n0 + (int)(threadIdx.x >> 1), N - 1);
-        sub_load<F>(W + (size_t)n * fmt_row_bytes_rt(F, K), K, (k0 >> 5) + (int)(threadIdx.x & 1), r);
-    }
-    __device__ __forceinline__ void store(uint4* Lb, int k0) const {
-        const int t = threadIdx.x, h = t & 1, row = t >> 1;
-        float w[32];
-        sub_decode<F>(r, (k0 >> 5) + h, w);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            uint32_t o[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) o[k] = f2bf_bits(w[8 * c + 2 * k]) | (f2bf_bits(w[8 * c + 2 * k + 1]) << 16);
-            Lb[swz(row, 4 * h + c)] = make_uint4(o[0], o[1], o[2], o[3]);
-        }
-    }
-};
-
-// D = A . W^T with W from the source WR (Q4_K blocks, bf16 rows or another format), f32 or bf16 (RNE)
-// out.  K % 128 == 0 (an even step count for the 3 x 2 stage unroll).
-template <class WR, bool OUT_BF16>
-__global__ void __launch_bounds__(kPPThreads) k_gemm_pp(const uint16_t* __restrict__ A, const uint8_t* __restrict__ W,
-                                                       void* __restrict__ Dv, int M, int N, int K, int ldd, int lda,
-                                                       int ldw) {
-    const int mt = (M + GBM - 1) / GBM, nt = (N + GBN - 1) / GBN;
-    int tm, tn;
-    tile_of(blockIdx.x, mt, nt, tm, tn);
-    const int m0 = tm * GBM, n0 = tn * GBN;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave & 1, wn = wave >> 1;
-    const int nk = K / GBK, lastk = (nk - 1) * GBK;
-    WR wr;
-    wr.load(W, N, K, ldw, n0, 0);
-    dma_a_pp(A, M, lda, m0, 0, ga<0>());
-    dma_a_pp(A, M, lda, m0, min(GBK, lastk), ga<1>());
-    wr.store(gb<0>(), 0);
-    wr.load(W, N, K, ldw, n0, min(GBK, lastk));
-    __builtin_amdgcn_s_waitcnt(0);
-    lds_barrier();
-    f32x16 acc[4][2];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int jn = 0; jn < 2; ++jn)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][jn][e] = 0.f;
-    const int fr = lane & 31, fc = lane >> 5, fx = (fr >> 1) & 7;
-    int foa[4], fob[4];
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-        foa[ks] = (128 * wm + fr) * 8 + ((2 * ks + fc) ^ fx);
-        fob[ks] = (64 * wn + fr) * 8 + ((2 * ks + fc) ^ fx);
-    }
-    // step s with A stage SA = s % 3 and W stage SB = s % 2
-    auto body = [&](auto sa_c, auto sb_c, int s) {
-        constexpr int SA = decltype(sa_c)::value, SB = decltype(sb_c)::value;
-        const uint4* La = ga<SA>();
-        const uint4* Lb = gb<SB>();
-        dma_a_pp(A, M, lda, m0, min((s + 2) * GBK, lastk), ga<(SA + 2) % 3>());
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            bf16x8 af[4], bf[2];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) { const uint4 v = La[foa[ks] + 256 * t]; af[t] = *(const bf16x8*)&v; }
-#pragma unroll
-            for (int t = 0; t < 2; ++t) { const uint4 v = Lb[fob[ks] + 256 * t]; bf[t] = *(const bf16x8*)&v; }
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int jn = 0; jn < 2; ++jn) acc[i][jn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i], bf[jn], acc[i][jn], 0, 0, 0);
-        }
-        wr.store(gb<1 - SB>(), min((s + 1) * GBK, lastk));
-        wr.load(W, N, K, ldw, n0, min((s + 2) * GBK, lastk));
-        // A tile s+1 (DMA'd a step ago, before W tile s+1's loads) has landed once at most this
-        // step's 4 DMAs and 3 W loads are outstanding
-        __builtin_amdgcn_s_waitcnt(0x0F77);   // vmcnt <= 7
-        lds_barrier_dma();
-    };
-    int s = 0;
-    for (; s + 6 <= nk; s += 6) {
-        body(IC<0>(), IC<0>(), s);
-        body(IC<1>(), IC<1>(), s + 1);
-        body(IC<2>(), IC<0>(), s + 2);
-        body(IC<0>(), IC<1>(), s + 3);
-        body(IC<1>(), IC<0>(), s + 4);
-        body(IC<2>(), IC<1>(), s + 5);
-    }
-    if (s < nk) {                              // nk is even, so 2 or 4 steps remain
-        body(IC<0>(), IC<0>(), s);
-        body(IC<1>(), IC<1>(), s + 1);
-        if (s + 2 < nk) {
-            body(IC<2>(), IC<0>(), s + 2);
-            body(IC<0>(), IC<1>(), s + 3);
-        }
-    }
-    __builtin_amdgcn_s_waitcnt(0);            // drain the clamped trailing DMAs
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const int m = m0 + 128 * wm + 32 * i + 8 * (e >> 2) + 4 * fc + (e & 3);
-            if (m >= M) continue;
-#pragma unroll
-            for (int jn = 0; jn < 2; ++jn) {
-                const int n = n0 + 64 * wn + 32 * jn + fr;
-                if (n < N) {
-                    if constexpr (OUT_BF16) ((uint16_t*)Dv)[(size_t)m * ldd + n] = (uint16_t)f2bf_bits(acc[i][jn][e]);
-                    else ((float*)Dv)[(size_t)m * ldd + n] = acc[i][jn][e];
-                }
-            }
-        }
-    }
+    return best;
 }
 
-// One workgroup of k_gemm_pp fills a CU (160 KiB of LDS), so its tiles run in rounds of one per
-// CU.  When the last round would keep at most a quarter of the CUs busy for a whole tile time, the
-// 256 x 256 kernel takes only whole rounds (whole columns of M tiles) and the remaining columns go
-// to the grouped-GEMM kernel as (32 rows x 256 columns) work units, enough of them to spread over
-// every CU.  Every output element is one bf16 MFMA dot product over K in the same order either way.
-int launch_gemm_q4k(const void* W, const uint16_t* A, float* D, int M, int N, int K, hipStream_t s) {
-    const int mt = (M + GBM - 1) / GBM, nt = (N + GBN - 1) / GBN, cus = device_cu_count();
-    int nbig = nt;                                   // column tiles for the 256 x 256 kernel
-    const int total = mt * nt, rem = total % cus;
-    if (total > cus && rem != 0 && 4 * rem <= cus && mt <= cus) nbig = (total - rem) / mt;
-    const int nb_cols = std::min(N, nbig * GBN);
-    if (nbig > 0) {
-        hipLaunchKernelGGL((k_gemm_pp<WRawQ4KHalf, false>), dim3(mt * nbig), dim3(kPPThreads), 0, s, A, (const uint8_t*)W, D, M,
-                           nb_cols, K, N, K, K);
-        QMM_LAUNCH_CHECK();
-    }
-    if (nb_cols < N) {
-        const size_t rowbytes = (size_t)(K / 256) * 144;
-        return launch_q4k_rows_gemm((const uint8_t*)W + (size_t)nb_cols * rowbytes, A, D + nb_cols, M, N - nb_cols, K, N, 32, s);
-    }
+template <int F, bool OUT_BF16, int NRB, int CW, int KS, int ST>
+int launch_tile(const GemmArgs& a, hipStream_t s) {
+    const int grid = tile_count(TileShape{NRB, CW, KS, 0, 0}, a.M, a.N);
+    hipLaunchKernelGGL((k_gemm_tile<F, NRB, CW, KS, ST, OUT_BF16>), dim3(grid), dim3(64 * CW * KS), 0, s, a);
+    QMM_LAUNCH_CHECK();
     return QMM_OK;
+}
+
+// D = A . W^T with W from source F, f32 or bf16 (RNE) out; K % 64 == 0
+template <int F, bool OUT_BF16>
+int launch_gemm(const GemmArgs& a, hipStream_t s) {
+    switch (pick_tile(a)) {
+        case 0: return launch_tile<F, OUT_BF16, 1, 1, 8, 4>(a, s);
+        case 1: return launch_tile<F, OUT_BF16, 2, 1, 8, 2>(a, s);
+        case 2: return launch_tile<F, OUT_BF16, 2, 2, 4, 4>(a, s);
+        case 3: return launch_tile<F, OUT_BF16, 4, 2, 4, 2>(a, s);
+        case 4: return launch_tile<F, OUT_BF16, 4, 4, 2, 4>(a, s);
+        case 5: return launch_tile<F, OUT_BF16, 4, 8, 1, 4>(a, s);
+        case 6: return launch_tile<F, OUT_BF16, 5, 8, 1, 4>(a, s);
+        case 7: return launch_tile<F, OUT_BF16, 6, 8, 1, 4>(a, s);
+        case 8: return launch_tile<F, OUT_BF16, 8, 8, 1, 4>(a, s);
+        default: return QMM_ERR_SHAPE;
+    }
 }
 
 
@@ -591,20 +388,20 @@ int qmm_gemm_wq(int fmt, const void* W, const uint16_t* A, float* D, int M, int 
         return QMM_ERR_FORMAT;
     if (!W || !A || !D) return QMM_ERR_NULL;
     // K % 256 for the block formats (K % 512 for Q6_K_SOA: an even block count keeps its streams dword
-    // aligned); the 32-weight SoA formats need K % 128 (the kernel's even step count)
+    // aligned), K % 128 for the 32-weight SoA formats
     const int kg = (fmt == QMM_Q8_0_SOA || fmt == QMM_Q5_1_SOA) ? 2 * GBK : fmt == QMM_Q6_K_SOA ? 512 : 256;
     if (M <= 0 || N <= 0 || K <= 0 || K % kg != 0) return QMM_ERR_SHAPE;
+    const size_t rb = fmt_row_bytes_rt(fmt, K);
+    const GemmArgs a{(const uint8_t*)A, (const uint8_t*)W, D, (uint32_t)K * 2u, (uint32_t)rb, (uint32_t)rb, M, N, K, N};
     hipStream_t s = (hipStream_t)stream;
-    if (fmt == QMM_Q4_K) return launch_gemm_q4k(W, A, D, M, N, K, s);
-    const dim3 grid((unsigned)(((M + GBM - 1) / GBM) * ((N + GBN - 1) / GBN)));
-#define QMM_GWQ(F) case F: hipLaunchKernelGGL((k_gemm_pp<WRawFmtHalf<F>, false>), grid, dim3(kPPThreads), 0, s, A, (const uint8_t*)W, \
-                                              (void*)D, M, N, K, N, K, K); break;
     switch (fmt) {
-        QMM_GWQ(QMM_Q5_K) QMM_GWQ(QMM_IQ4_XS) QMM_GWQ(QMM_Q6_K_SOA) QMM_GWQ(QMM_Q8_0_SOA) QMM_GWQ(QMM_Q5_1_SOA)
+        case QMM_Q4_K: return launch_gemm<QMM_Q4_K, false>(a, s);
+        case QMM_Q5_K: return launch_gemm<QMM_Q5_K, false>(a, s);
+        case QMM_IQ4_XS: return launch_gemm<QMM_IQ4_XS, false>(a, s);
+        case QMM_Q6_K_SOA: return launch_gemm<QMM_Q6_K_SOA, false>(a, s);
+        case QMM_Q8_0_SOA: return launch_gemm<QMM_Q8_0_SOA, false>(a, s);
+        default: return launch_gemm<QMM_Q5_1_SOA, false>(a, s);
     }
-#undef QMM_GWQ
-    QMM_LAUNCH_CHECK();
-    return QMM_OK;
 }
 
 int qmm_gemm_bf16_ld(const uint16_t* A, int lda, const uint16_t* W, int ldw, uint16_t* D, int M, int N, int K, void* stream) {
@@ -614,13 +411,12 @@ int qmm_gemm_bf16_ld(const uint16_t* A, int lda, const uint16_t* W, int ldw, uin
     if (((uintptr_t)A | (uintptr_t)W) % 16 != 0 || lda % 8 != 0 || ldw % 8 != 0) return QMM_ERR_ARG;
     // the DMA of A addresses rows with 32-bit element offsets
     if ((uint64_t)(M - 1) * (uint64_t)lda + (uint64_t)K > 0xffffffffull) return QMM_ERR_SHAPE;
+    const GemmArgs a{(const uint8_t*)A, (const uint8_t*)W, D, (uint32_t)lda * 2u, (uint32_t)ldw * 2u, (uint32_t)K * 2u, M, N, K, N};
+    if (pick_tile(a) >= 0) return launch_gemm<QMM_W_BF16, true>(a, (hipStream_t)stream);
+    // rows so far apart that no tile's span fits a buffer resource
     const int grid = ((M + GBM - 1) / GBM) * ((N + GBN - 1) / GBN);
-    if (K % (2 * GBK) == 0)     // the two-waves-per-SIMD kernel of the fused GEMM, bf16 rows as its W source
-        hipLaunchKernelGGL((k_gemm_pp<WRawBf16Half, true>), dim3(grid), dim3(kPPThreads), 0, (hipStream_t)stream, A,
-                           (const uint8_t*)W, (void*)D, M, N, K, N, lda, ldw);
-    else
-        hipLaunchKernelGGL((k_gemm<BLoadBf16, uint16_t, true>), dim3(grid), dim3(256), kGemmLds, (hipStream_t)stream, A, W,
-                           (void*)D, M, N, K, lda, ldw);
+    hipLaunchKernelGGL((k_gemm<BLoadBf16, uint16_t, true>), dim3(grid), dim3(256), kGemmLds, (hipStream_t)stream, A, W, (void*)D, M, N,
+                       K, lda, ldw);
     QMM_LAUNCH_CHECK();
     return QMM_OK;
 }

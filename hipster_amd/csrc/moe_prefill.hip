@@ -345,8 +345,7 @@ struct XArgs {
     void* D;               // f32 [k][ldd], or bf16 h [k][ldd] in gate/up mode
     int N, K, nb;          // nb = weight-row blocks per tile
     int ldd;               // row stride of D (elements)
-    int trows, nimp, M;    // tiles == nullptr: implicit tiles of trows rows of expert 0, nimp of them, M rows;
-                           // otherwise nimp = capacity of tiles (the device count is clamped to it)
+    int cap;               // capacity of tiles (the device count is clamped to it)
     int bpu;               // k_moe_gemm_as: 256-row weight blocks per work unit
 };
 
@@ -588,10 +587,8 @@ __global__ void __launch_bounds__(XTHREADS) k_moe_gemm_x(XArgs a) {
     __shared__ int rows[XBM];
     const int id = blockIdx.x, sid = id >> 3;
     const int tix = 8 * (sid / a.nb) + (id & 7), nbi = sid % a.nb;
-    if (tix >= (a.tiles ? min(a.counts[0] + a.counts[1], a.nimp) : a.nimp)) return;
-    qmm_moe_tile tl;
-    if (a.tiles) tl = a.tiles[tix];
-    else tl = qmm_moe_tile{0, tix * a.trows, min(a.trows, a.M - tix * a.trows)};
+    if (tix >= min(a.counts[0] + a.counts[1], a.cap)) return;
+    qmm_moe_tile tl = a.tiles[tix];
     tl.ncols = max(1, min(tl.ncols, XBM));
     if (threadIdx.x < XBM) {
         const int k = tl.k0 + min((int)threadIdx.x, tl.ncols - 1);
@@ -790,7 +787,7 @@ __global__ void __launch_bounds__(kAsThreads) k_moe_gemm_as(XArgs a) {
     const int nu = (a.nb + a.bpu - 1) / a.bpu;
     const int id = blockIdx.x, sid = id >> 3;
     const int tix = 8 * (sid / nu) + (id & 7), ui = sid % nu;
-    if (tix >= min(a.counts[0] + a.counts[1], a.nimp)) return;
+    if (tix >= min(a.counts[0] + a.counts[1], a.cap)) return;
     qmm_moe_tile tl = a.tiles[tix];
     tl.ncols = max(1, min(tl.ncols, XBM));
     if (threadIdx.x < XBM) {
@@ -816,13 +813,6 @@ int launch_moe_gemm_as(XArgs a, int max_tiles, hipStream_t s) {
 }
 
 }  // namespace
-
-int launch_q4k_rows_gemm(const void* W, const uint16_t* A, float* D, int M, int N, int K, int ldd, int trows, hipStream_t s) {
-    const int nimp = (M + trows - 1) / trows;
-    XArgs a{(const uint8_t*)W, (const uint8_t*)W, nullptr, nullptr, 0, nullptr, nullptr, nullptr, A, D, N, K,
-            (N + XBW - 1) / XBW, ldd, trows, nimp, M};
-    return launch_moe_gemm_x(false, a, nimp, s);
-}
 
 namespace {
 
@@ -887,7 +877,7 @@ int qmm_moe_gemm_bf16(int fmt, int shared_fmt, const void* W, const void* Wsh, s
         return launch_moe_gemm_fmt(fmt, shared_fmt, W, Wsh, ebytes, tiles, counts, max_tiles, rowtab, A, D, N, K,
                                    (hipStream_t)stream);
     XArgs a{(const uint8_t*)W, (const uint8_t*)Wsh, nullptr, nullptr, ebytes, tiles, counts, rowtab, A, D, N, K,
-            (N + XBW - 1) / XBW, N, 0, max_tiles, 0, kAsBlocksPerUnit};
+            (N + XBW - 1) / XBW, N, max_tiles, kAsBlocksPerUnit};
     if (K == kAsK) return launch_moe_gemm_as(a, max_tiles, (hipStream_t)stream);
     return launch_moe_gemm_x(false, a, max_tiles, (hipStream_t)stream);
 }
@@ -900,7 +890,7 @@ int qmm_moe_gemm_gate_up_bf16(int fmt, int shared_fmt, const void* Wg, const voi
     if (N <= 0 || K <= 0 || K % 256 != 0 || max_tiles < 0) return QMM_ERR_SHAPE;
     if (max_tiles == 0) return QMM_OK;
     XArgs a{(const uint8_t*)Wg, (const uint8_t*)Wgsh, (const uint8_t*)Wu, (const uint8_t*)Wush, ebytes, tiles, counts,
-            rowtab, A, H, N, K, (N + XBW / 2 - 1) / (XBW / 2), N, 0, max_tiles, 0};
+            rowtab, A, H, N, K, (N + XBW / 2 - 1) / (XBW / 2), N, max_tiles, 0};
     return launch_moe_gemm_x(true, a, max_tiles, (hipStream_t)stream);
 }
 

@@ -1,0 +1,77 @@
+"""The tile kernel of the prefill GEMMs (gemm_tile.hpp) where its tilings can go wrong: every weight
+source, sizes around the edges of each tile (rows 32, 64, 128, 192; columns 32, 64, 128, 256), K steps that do not
+divide among the K groups, one row, one column, and a shape per tile choice.
+
+Bound: every product of two bf16 values is exact in f32, so only the K additions round.  Their errors add
+up as a random walk, each at most 2^-24 of a partial sum that grows like sqrt(k): sqrt(K) 2^-24 relative
+in the 2-norm, against the float64 product of the same bf16 operands."""
+import numpy as np
+import pytest
+import torch
+
+from hipster_amd import qmm, synth
+from tests.gpu_util import dev
+
+pytestmark = pytest.mark.gpu
+SHAPES = [(1, 70, 512), (70, 1, 512), (17, 33, 1536), (33, 1024, 2560), (40, 6144, 1024), (65, 63, 512), (129, 257, 1024), (300, 2500, 512),
+          (193, 8200, 512), (385, 17000, 512), (1100, 300, 1536), (2048, 5120, 512)]
+
+
+def operands(fmt, M, N, K, seed):
+    A = torch.from_numpy(synth.normal_f32(seed, (M, K))).cuda().bfloat16()
+    W = dev(synth.matrix(seed + 1, fmt, N, K))
+    Wb = torch.zeros((N, K), dtype=torch.int16, device="cuda")
+    qmm.dequant_bf16(fmt, W, Wb, N, K)
+    Wb = Wb.view(torch.bfloat16)
+    return A, W, Wb, A.double() @ Wb.double().t()
+
+
+def err(got, ref):
+    return ((got.double() - ref).norm() / ref.norm()).item()
+
+
+@pytest.mark.parametrize("fmt", [synth.Q4_K, synth.Q5_K, synth.IQ4_XS, synth.Q6_K_SOA, synth.Q8_0_SOA, synth.Q5_1_SOA])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_gemm_wq_tiles(gpu, fmt, M, N, K):
+    A, W, Wb, ref = operands(fmt, M, N, K, 7000 + M + N)
+    D = torch.full((M, N), float("nan"), device="cuda")
+    qmm.gemm_wq(fmt, W, A, D, M, N, K)
+    assert err(D, ref) <= K ** 0.5 * 2.0 ** -24
+    # the bf16 GEMM takes the same tile and K order, but lanes of some formats hold k in another order: the same
+    # sums within the bound, then one rounding to bf16 (8 bits: 2^-8 at most)
+    Db = torch.zeros((M, N), dtype=torch.bfloat16, device="cuda")
+    qmm.gemm_bf16(A, Wb, Db, M, N, K)
+    assert err(Db, ref) <= 2.0 ** -8
+
+
+@pytest.mark.parametrize("fmt,K", [(synth.Q8_0_SOA, 128), (synth.Q5_1_SOA, 640), (synth.Q4_K, 256), (synth.Q6_K_SOA, 512)])
+def test_gemm_wq_short_k(gpu, fmt, K):
+    """fewer K steps than K groups, and a last group without a step"""
+    A, W, Wb, ref = operands(fmt, 21, 70, K, 7100 + K)
+    D = torch.full((21, 70), float("nan"), device="cuda")
+    qmm.gemm_wq(fmt, W, A, D, 21, 70, K)
+    assert err(D, ref) <= K ** 0.5 * 2.0 ** -24
+
+
+def test_gemm_bf16_odd_step_count_and_strides(gpu):
+    """K = 192 (three steps) and operands that are views of wider matrices, garbage (NaN) around them"""
+    M, N, K = 45, 300, 192
+    A = torch.full((M, 256), float("nan"), device="cuda", dtype=torch.bfloat16)
+    W = torch.full((N, 200), float("nan"), device="cuda", dtype=torch.bfloat16)
+    A[:, :K] = torch.from_numpy(synth.normal_f32(7200, (M, K))).cuda().bfloat16()
+    W[:, :K] = torch.from_numpy(synth.normal_f32(7201, (N, K))).cuda().bfloat16()
+    D = torch.zeros((M, N), dtype=torch.bfloat16, device="cuda")
+    qmm.gemm_bf16_ld(A, 256, W, 200, D, M, N, K)
+    assert err(D, A[:, :K].double() @ W[:, :K].double().t()) <= 2.0 ** -8
+
+
+def test_gemm_wq_rows_do_not_mix(gpu):
+    """an infinite activation spoils its own row only, also beside rows and K steps that a tile pads"""
+    M, N, K = 40, 96, 768
+    A, W, Wb, ref = operands(synth.Q4_K, M, N, K, 7300)
+    A[7, 5] = float("inf")
+    D = torch.zeros((M, N), device="cuda")
+    qmm.gemm_wq(synth.Q4_K, W, A, D, M, N, K)
+    keep = np.arange(M) != 7
+    assert not torch.isfinite(D[7]).any()
+    assert err(D[keep], ref[torch.from_numpy(keep)]) <= K ** 0.5 * 2.0 ** -24
