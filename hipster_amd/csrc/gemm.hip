@@ -261,14 +261,14 @@ __global__ void __launch_bounds__(256) k_gemm(const uint16_t* __restrict__ A, co
 }
 // ------------------------------------------------------------------------------------------
 // Tile choice of the dequantising GEMM (gemm_tile.hpp).  A workgroup fills a CU, so a shape takes
-// ceil(tiles / CUs) rounds of ceil(K / 64 / KS) steps each, and the choice is the tile with the least
+// ceil(tiles / CUs) rounds of about K / 64 / KS steps each, and the choice is the tile with the least
 // rounds x (steps x step time + launch and reduction).  Step times in 0.01 us, measured with Q4_K weights on
 // 256 CUs: large tiles do the most work per step (192 x 256: 34 blocks of 32 x 32 x 64 per us, 32 x 32 with
 // eight K groups: 9) and small ones fill the chip where M x N is small.  The choice does not look at the
 // format, so every weight source gets the same K order.
 struct TileShape { int nrb, cw, ks, step, fixed; };
-constexpr TileShape kTiles[] = {{1, 1, 8, 90, 400}, {2, 1, 8, 125, 500}, {2, 2, 4, 87, 500}, {4, 2, 4, 116, 600}, {4, 4, 2, 102, 600},
-                                {4, 8, 1, 98, 600}, {5, 8, 1, 122, 600}, {6, 8, 1, 139, 600}, {8, 8, 1, 156, 600}};
+constexpr TileShape kTiles[] = {{1, 1, 8, 75, 200}, {2, 1, 8, 110, 250}, {2, 2, 4, 75, 200}, {4, 2, 4, 120, 300}, {4, 4, 2, 105, 300},
+                                {4, 8, 1, 90, 400}, {5, 8, 1, 108, 400}, {6, 8, 1, 129, 400}, {8, 8, 1, 150, 400}};
 constexpr int kNumTiles = (int)(sizeof(kTiles) / sizeof(kTiles[0]));
 
 int tile_count(const TileShape& t, int M, int N) {
@@ -289,7 +289,7 @@ int pick_tile(const GemmArgs& a) {
         const TileShape& t = kTiles[i];
         if (!tile_fits(t, a)) continue;
         const long long rounds = (tile_count(t, a.M, a.N) + cus - 1) / cus;
-        const long long c = rounds * ((long long)((nk + t.ks - 1) / t.ks) * t.step + t.fixed);
+        const long long c = rounds * ((long long)gt_local_steps(nk, t.ks) * t.step + t.fixed);
         if (best < 0 || c < cost) { best = i; cost = c; }
     }
     return best;
@@ -315,7 +315,8 @@ int launch_gemm(const GemmArgs& a, hipStream_t s) {
         case 5: return launch_tile<F, OUT_BF16, 4, 8, 1, 4>(a, s);
         case 6: return launch_tile<F, OUT_BF16, 5, 8, 1, 4>(a, s);
         case 7: return launch_tile<F, OUT_BF16, 6, 8, 1, 4>(a, s);
-        case 8: return launch_tile<F, OUT_BF16, 8, 8, 1, 4>(a, s);
+        // bf16 rows: four steps' weights (64 registers) beside 128 accumulators would spill
+        case 8: return launch_tile<F, OUT_BF16, 8, 8, 1, F == QMM_W_BF16 ? 2 : 4>(a, s);
         default: return QMM_ERR_SHAPE;
     }
 }
