@@ -5,15 +5,20 @@
 //   D[k0 + r][n] = sum_k A[rowtab[k0 + r]][k] * bf16(W_e[n][k])      (f32 out, sorted row order)
 // with W_e dequantised exactly (the arithmetic of qmm_dequant_bf16) and bf16 MFMA, f32 accumulation.
 //
-// Workgroup = (tile, 128 weight rows), 256 threads = 4 waves.  Wave w owns the block's weight rows
-// 32w..32w+31 (one v_mfma_f32_32x32x16_bf16 column block) and the tile's NRB row blocks of 32.  The K
-// loop steps by 32 -- one sub-block, the scale granule of every format: threads 0-127 dequantise
-// their weight row's sub-block to bf16 and threads 128-255 copy the tile's 128 A rows of the step,
-// both into the LDS stage that the next step's MFMAs read, while this step's MFMAs run from the
-// other stage (one barrier per step); the raw bytes are loaded a step before that.  Stage rows are
-// 80 bytes apart (32 bf16 + 16 bytes of padding: the 16-byte fragment reads of a half-wave's 32 rows
-// spread over the banks).
+// Workgroup = (tile, 128 weight rows), 256 threads = 4 waves, the core of gemm_tile.hpp with the tile's
+// ceil(rows / 32) row blocks.  One K group and four stages: of the shapes measured (128 or 256 columns, 1, 2 or 4 K
+// groups, two or four stages) the best at 64, 600 and 2048 tokens.  Weights are read once a tile; with the 32-k
+// steps through LDS of k_moe_gemm_fmt before it, waiting for its loads at every step, the calls took
+// (512 experts, Zipf routing, HIP graph replay, gate Q5_K 640 x 2560 / down Q5_1 2560 x 640):
+//   64 tokens 134 / 78 -> 37 / 35 us,  600 tokens 225 / 207 -> 82 / 107 us,  2048 tokens 368 / 366 -> 153 / 212 us
+//
+// k_moe_gemm_fmt stays for Q5_1 rows of an odd number of 32-weight blocks, which steps of 64 do not divide: its K
+// loop steps by 32, threads 0-127 dequantise their weight row's sub-block to bf16 and threads 128-255 copy the tile's
+// 128 A rows of the step, both into the LDS stage that the next step's MFMAs read (one barrier per step; the raw bytes
+// are loaded a step before that).  Stage rows are 80 bytes apart (32 bf16 + 16 bytes of padding: the 16-byte fragment
+// reads of a half-wave's 32 rows spread over the banks).
 #include "fmt_dequant.hpp"
+#include "gemm_tile.hpp"
 #include "qmm_common.hpp"
 
 namespace qmm {
@@ -119,24 +124,30 @@ __device__ __forceinline__ void fmt_tile(const FArgs& a, const qmm_moe_tile tl, 
 // format, as the reference launches its routed and shared tiles apart: part 0 takes the routed
 // tiles [0, counts[0]), part 1 the shared ones [counts[0], counts[0] + counts[1]), part 2 both
 // (one format for all).  Tiles past the device count (clamped to the capacity) exit at once.
-template <int F>
-__global__ void __launch_bounds__(256) k_moe_gemm_fmt(FArgs a, int part) {
-    __shared__ __align__(16) uint16_t st[2 * kFStage];
-    __shared__ int rows[FBM];
+__device__ __forceinline__ bool fmt_unit(const FArgs& a, int part, int* rows, qmm_moe_tile& tl, int& n0) {
     const int id = blockIdx.x, sid = id >> 3;
     const int local = 8 * (sid / a.nb) + (id & 7), nbi = sid % a.nb;
     const int c0 = a.counts[0], c1 = a.counts[1];
     const int first = part == 1 ? c0 : 0, count = part == 0 ? c0 : part == 1 ? c1 : c0 + c1;
     const int tix = first + local;
-    if (local >= count || tix >= a.nimp) return;
-    qmm_moe_tile tl = a.tiles[tix];
+    if (local >= count || tix >= a.nimp) return false;
+    tl = a.tiles[tix];
     tl.ncols = max(1, min(tl.ncols, FBM));
     if (threadIdx.x < FBM) {
         const int k = tl.k0 + min((int)threadIdx.x, tl.ncols - 1);
         rows[threadIdx.x] = a.rowtab ? a.rowtab[k] : k;
     }
     __syncthreads();
-    const int n0 = nbi * FBN;
+    n0 = nbi * FBN;
+    return true;
+}
+template <int F>
+__global__ void __launch_bounds__(256) k_moe_gemm_fmt(FArgs a, int part) {
+    __shared__ __align__(16) uint16_t st[2 * kFStage];
+    __shared__ int rows[FBM];
+    qmm_moe_tile tl;
+    int n0;
+    if (!fmt_unit(a, part, rows, tl, n0)) return;
     switch ((tl.ncols + 31) >> 5) {
         case 1: fmt_tile<1, F>(a, tl, n0, st, rows); break;
         case 2: fmt_tile<2, F>(a, tl, n0, st, rows); break;
@@ -145,13 +156,74 @@ __global__ void __launch_bounds__(256) k_moe_gemm_fmt(FArgs a, int part) {
     }
 }
 
+// A tile with a row beyond the span of a 32-bit buffer offset (an A of more than 3.75 GiB): each thread sums whole
+// output elements, straight from memory
+constexpr uint32_t kASpan = 0xf0000000u;
+template <int F>
+__device__ void moe_tile_far(const FArgs& a, const qmm_moe_tile& tl, const uint8_t* wb, size_t ldw, int n0, int nn, const int* rows) {
+    for (int i = threadIdx.x; i < tl.ncols * nn; i += blockDim.x) {
+        const int r = i / nn, n = i - r * nn;
+        const uint16_t* x = a.A + (size_t)rows[r] * a.K;
+        float acc = 0.f;
+        for (int sb = 0; sb < a.K / 32; ++sb) {
+            float w[32];
+            dq_sub32<F>(wb + (size_t)n * ldw, a.K, sb, w);
+            for (int k = 0; k < 32; ++k) acc = __builtin_fmaf(bf2f(x[32 * sb + k]), bf2f(f2bf_bits(w[k])), acc);
+        }
+        a.D[(size_t)(tl.k0 + r) * a.N + n0 + n] = acc;
+    }
+}
+
+// The grouped GEMM on gemm_tile.hpp's core (K % 64 == 0).  Workgroup = (tile, 32 CW weight rows).
+template <int F>
+__device__ __forceinline__ void moe_tile_unit(const FArgs& a, int part) {
+    constexpr int kStage = FBM * 8;
+    __shared__ uint4 s0[kStage], s1[kStage], s2[kStage], s3[kStage];
+    __shared__ int rows[FBM];
+    qmm_moe_tile tl;
+    int n0;
+    if (!fmt_unit(a, part, rows, tl, n0)) return;
+    const int lane = threadIdx.x & 63, h = lane >> 5;
+    const int n = n0 + 32 * (int)(threadIdx.x >> 6) + (lane & 31);
+    const uint32_t lda = 2u * (uint32_t)a.K, ldw = (uint32_t)fmt_row_bytes_rt(F, a.K);
+    const uint8_t* wb = (tl.expert < 0 ? a.wsh : a.w + (size_t)tl.expert * a.ebytes) + (size_t)n0 * ldw;
+    const uint32_t wbytes = (uint32_t)min(FBN, a.N - n0) * ldw;
+    const bool far = threadIdx.x < FBM && ((unsigned long long)(unsigned)rows[threadIdx.x] + 1) * lda > kASpan;
+    if (__syncthreads_or(far)) {
+        moe_tile_far<F>(a, tl, wb, ldw, n0, min(FBN, a.N - n0), rows);
+        return;
+    }
+    auto go = [&](auto nrb_c) {
+        constexpr int NRB = decltype(nrb_c)::value;
+        gemm_tile_core<F, NRB, FBN / 32, 1, 4>(
+            s0, s1, s2, s3, (const uint8_t*)a.A, kASpan, wb, wbytes, ldw, a.K,
+            [&](int r) { return r < tl.ncols ? (uint32_t)rows[r] * lda : kASpan + 0x08000000u; },   // past the span: zeros
+            [&](int i, int e, float v) {
+                const int r = 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
+                if (r < tl.ncols && n < a.N) a.D[(size_t)(tl.k0 + r) * a.N + n] = v;
+            });
+    };
+    switch ((tl.ncols + 31) >> 5) {
+        case 1: go(std::integral_constant<int, 1>()); break;
+        case 2: go(std::integral_constant<int, 2>()); break;
+        case 3: go(std::integral_constant<int, 3>()); break;
+        default: go(std::integral_constant<int, 4>()); break;
+    }
+}
+template <int F>
+__global__ void __launch_bounds__(256) k_moe_gemm_tile(FArgs a, int part) {
+    moe_tile_unit<F>(a, part);
+}
+
 int launch_fmt_part(int fmt, const FArgs& a, int part, int grid, hipStream_t s) {
     switch (fmt) {
-        case QMM_Q4_K: hipLaunchKernelGGL(k_moe_gemm_fmt<QMM_Q4_K>, dim3(grid), dim3(256), 0, s, a, part); break;
-        case QMM_Q5_K: hipLaunchKernelGGL(k_moe_gemm_fmt<QMM_Q5_K>, dim3(grid), dim3(256), 0, s, a, part); break;
-        case QMM_IQ4_XS: hipLaunchKernelGGL(k_moe_gemm_fmt<QMM_IQ4_XS>, dim3(grid), dim3(256), 0, s, a, part); break;
-        case QMM_Q8_0_SOA: hipLaunchKernelGGL(k_moe_gemm_fmt<QMM_Q8_0_SOA>, dim3(grid), dim3(256), 0, s, a, part); break;
-        default: hipLaunchKernelGGL(k_moe_gemm_fmt<QMM_Q5_1_SOA>, dim3(grid), dim3(256), 0, s, a, part); break;
+        case QMM_Q4_K: hipLaunchKernelGGL(k_moe_gemm_tile<QMM_Q4_K>, dim3(grid), dim3(256), 0, s, a, part); break;
+        case QMM_Q5_K: hipLaunchKernelGGL(k_moe_gemm_tile<QMM_Q5_K>, dim3(grid), dim3(256), 0, s, a, part); break;
+        case QMM_IQ4_XS: hipLaunchKernelGGL(k_moe_gemm_tile<QMM_IQ4_XS>, dim3(grid), dim3(256), 0, s, a, part); break;
+        case QMM_Q8_0_SOA: hipLaunchKernelGGL(k_moe_gemm_tile<QMM_Q8_0_SOA>, dim3(grid), dim3(256), 0, s, a, part); break;
+        default:
+            if (a.K % 64 == 0) hipLaunchKernelGGL(k_moe_gemm_tile<QMM_Q5_1_SOA>, dim3(grid), dim3(256), 0, s, a, part);
+            else hipLaunchKernelGGL(k_moe_gemm_fmt<QMM_Q5_1_SOA>, dim3(grid), dim3(256), 0, s, a, part);
     }
     QMM_LAUNCH_CHECK();
     return QMM_OK;

@@ -75,3 +75,28 @@ def test_gemm_wq_rows_do_not_mix(gpu):
     keep = np.arange(M) != 7
     assert not torch.isfinite(D[7]).any()
     assert err(D[keep], ref[torch.from_numpy(keep)]) <= K ** 0.5 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("fmt,N,K", [(synth.Q4_K, 130, 256), (synth.Q5_K, 128, 512), (synth.IQ4_XS, 33, 768), (synth.Q8_0_SOA, 257, 192),
+                                     (synth.Q5_1_SOA, 2560, 640), (synth.Q5_1_SOA, 100, 96), (synth.Q8_0_SOA, 40, 64)])
+@pytest.mark.parametrize("gather", [True, False])
+def test_grouped_tiles(gpu, fmt, N, K, gather):
+    """every number of row blocks (tiles of 1, 31, 32, 33, 64, 65, 97, 128 rows), partial column blocks, K of a
+    partial chunk of steps (Q8_0 K = 64 and 192) and Q5_1 rows that steps of 64 do not divide, routed and shared tiles"""
+    sizes = [1, 31, 32, 33, 64, 65, 97, 128]
+    E, rows = len(sizes) - 1, sum(sizes)
+    sf = synth.Q8_0_SOA if fmt != synth.Q8_0_SOA and K % 64 == 0 else fmt
+    W, S = dev(synth.experts(7400 + K, fmt, E, N, K)), dev(synth.matrix(7401 + K, sf, N, K))
+    deq = lambda f, w: (lambda o: (qmm.dequant_bf16(f, w, o, N, K), o.view(torch.bfloat16).double())[1])(   # noqa: E731
+        torch.zeros((N, K), dtype=torch.int16, device="cuda"))
+    starts = np.concatenate([[0], np.cumsum(sizes)[:-1]])
+    tiles = np.array([[e, starts[e], sizes[e]] for e in range(E)] + [[-1, starts[E], sizes[E]]], np.int32)
+    A = torch.from_numpy(synth.normal_f32(7402, (rows if not gather else 200, K))).cuda().bfloat16()
+    rt = synth.rng(7403).integers(0, A.shape[0], rows).astype(np.int32) if gather else None
+    D = torch.full((rows, N), float("nan"), device="cuda")
+    qmm.moe_gemm_bf16(fmt, sf, W, S, W[0].numel(), dev(tiles), dev(np.array([E, 1], np.int32)), E + 1,
+                      dev(rt) if gather else None, A, D, N, K)
+    idx = torch.from_numpy(rt.astype(np.int64)).cuda() if gather else torch.arange(rows, device="cuda")
+    for e, (k0, n) in enumerate(zip(starts, sizes)):
+        ref = A[idx[k0:k0 + n]].double() @ (deq(fmt, W[e]) if e < E else deq(sf, S)).t()
+        assert err(D[k0:k0 + n], ref) <= K ** 0.5 * 2.0 ** -24, (e, n)
