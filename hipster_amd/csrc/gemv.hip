@@ -837,6 +837,11 @@ __device__ __forceinline__ void stage_f32_pairs(uint8_t* lds, int K, const XStag
     }
 }
 
+// explicit fused multiply-adds: both kernels below give a pair the same bits
+__device__ __forceinline__ float f32_pair_value(float dA, float sa, float dB, float sb, float mA, float xa, float mB, float xb) {
+    return __builtin_fmaf(dA, sa, __builtin_fmaf(dB, sb, -__builtin_fmaf(mA, xa, mB * xb)));
+}
+
 template <int NCOL, int NITER>
 __global__ void __launch_bounds__(kBlock) k_gemv_q4k_f32p(const uint8_t* __restrict__ W, const float* __restrict__ x,
                                                           float* __restrict__ y, int N, int K) {
@@ -888,7 +893,7 @@ __global__ void __launch_bounds__(kBlock) k_gemv_q4k_f32p(const uint8_t* __restr
                 sb = __builtin_fmaf(xb.w, (float)(hi >> 24), sb);
             }
             const float2 xs = *(const float2*)(xc + (size_t)K * 4 + (size_t)tk * 8);
-            const float v = dA * sa + dB16 * sb - (mA * xs.x + mB * xs.y);
+            const float v = f32_pair_value(dA, sa, dB16, sb, mA, xs.x, mB, xs.y);
             acc[c] += task < ntask ? v : 0.f;
         }
     }
@@ -910,6 +915,160 @@ int launch_q4k_f32p(const void* W, const float* x, float* y, int N, int K, hipSt
         default: return QMM_ERR_SHAPE;
     }
 #undef QMM_FP
+    QMM_LAUNCH_CHECK();
+    return QMM_OK;
+}
+
+// The same arithmetic for 2 to 4 columns on the f32 matrix cores.  v_mfma_f32_4x4x1 is sixteen independent 4 x 4
+// outer products: with the four rows of a wave's row group as columns and the four x columns as rows, block
+// t of it adds x[c][k] * q[row][k] of pair task t to all sixteen sums of the block, so a lane supplies its own row's
+// weight and one x value and gets four columns' sums.  Per weight that is one conversion and a quarter of an
+// LDS read of 16 bytes, where k_gemv_q4k_f32p reads x once per column and adds on the VALU.  Every sum is the same chain
+// of fused multiply-adds over k, so a column's bits are those of k_gemv_q4k_f32p.
+// One workgroup of eight waves per CU stages x (four columns of f32: 84 KiB at K = 5120) once and walks the row
+// groups, each wave loading its next group's weights while it computes.  Columns start 64 bytes apart modulo
+// the 256 of a bank round, so the four columns' reads of four pairs fill one round.  The matrix instruction's
+// rate bounds it (about 32 cycles for 256 multiply-adds here): 17408 x 5120 at four columns 49.3 -> 27.5 us.
+typedef float f32x4m __attribute__((ext_vector_type(4)));
+constexpr int kF32mBlock = 512;
+__host__ __device__ inline size_t f32m_col_bytes(int K) {
+    const size_t b = (size_t)K * 4 + (size_t)(K >> 3);
+    return (b + 255) / 256 * 256 + 64;
+}
+
+template <int NITER>
+__global__ void __launch_bounds__(kF32mBlock) k_gemv_q4k_f32m(const uint8_t* __restrict__ W, const float* __restrict__ x,
+                                                              float* __restrict__ y, int N, int K, int ncol) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int nb = K >> 8, ntask = 4 * nb, kp = K >> 6, ngrp = (N + 3) >> 2;
+    const size_t cs = f32m_col_bytes(K);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int t = lane >> 2, j = t & 3, r = lane & 3;          // pair task (+ 16 i), its place in the block, row of the group
+    const int step = (int)gridDim.x * (kF32mBlock / 64);
+    int g = (int)blockIdx.x + (int)gridDim.x * wave;            // few row groups spread over all CUs
+    auto rowp = [&](int grp) { return W + (size_t)min(4 * grp + r, N - 1) * ((size_t)nb * 144); };
+    Q4kPairs<NITER> A;
+    {   // x: all loads, then the first group's weights, then x to LDS (transposed in 16-byte units as
+        // stage_f32_pairs, with the 32-element sums behind each column)
+        constexpr int U = (NITER * 16 * 64 * 4 / 8 + kF32mBlock - 1) / kF32mBlock;
+        const int k8 = K >> 3, n8 = ncol * k8;
+        float4 v[U][2];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const float4* src = (const float4*)(x + 8 * (size_t)min((int)threadIdx.x + kF32mBlock * u, n8 - 1));
+            v[u][0] = src[0];
+            v[u][1] = src[1];
+        }
+        q4k_load_pairs<NITER>(rowp(min(g, ngrp - 1)), t, j, ntask, 0, A);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int e = (int)threadIdx.x + kF32mBlock * u;      // floats 8e..8e+7 (quads share e < n8)
+            const float4 a = v[u][0], b = v[u][1];
+            float sum = ((a.x + a.y) + (a.z + a.w)) + ((b.x + b.y) + (b.z + b.w));
+            sum += __int_as_float(quad_xor<1>(__float_as_int(sum)));
+            sum += __int_as_float(quad_xor<2>(__float_as_int(sum)));
+            if (e < n8) {
+                const int c = e / k8, f8 = e - c * k8, p = f8 >> 3, uu = 2 * (f8 & 7);
+                uint8_t* base = smem + (size_t)c * cs;
+                *(float4*)(base + (size_t)(uu * kp + p) * 16) = a;
+                *(float4*)(base + (size_t)((uu + 1) * kp + p) * 16) = b;
+                if ((f8 & 3) == 0) *(float*)(base + (size_t)K * 4 + (size_t)(f8 >> 2) * 4) = sum;
+            }
+        }
+        lds_barrier();
+    }
+    const Q4kPairDecode dc(j);
+    const uint8_t* xc = smem + (size_t)min(r, ncol - 1) * cs;      // the x column that this lane feeds
+    for (; g < ngrp; g += step) {
+        const uint8_t* np = rowp(min(g + step, ngrp - 1));
+        // All tasks side by side, 4 k at a time: a task's two chains wait for each of their matrix instructions, the
+        // 2 NITER chains of the row hide that and the LDS reads (x of the next 4 k is read ahead).  The next group's
+        // weights are loaded into the registers that this one is done with.
+        f32x4m sa[NITER], sb[NITER];
+        float4 xa[2][NITER], xb[2][NITER];
+        auto xread = [&](int q) {
+#pragma unroll
+            for (int i = 0; i < NITER; ++i) {
+                const uint8_t* xp = xc + (size_t)min(t + 16 * i, ntask - 1) * 16;
+                xa[q & 1][i] = *(const float4*)(xp + (size_t)(q * kp) * 16);
+                xb[q & 1][i] = *(const float4*)(xp + (size_t)((8 + q) * kp) * 16);
+            }
+        };
+        auto wread = [&](int part) {
+#pragma unroll
+            for (int i = 0; i < NITER; ++i) {
+                const uint8_t* bp = np + (size_t)(min(t + 16 * i, ntask - 1) >> 2) * 144;
+                if (part == 0) A.q0[i] = ld16(bp + 16 + 32 * j);
+                else if (part == 1) A.q1[i] = ld16(bp + 32 + 32 * j);
+                else A.h[i] = ld16(bp);
+            }
+        };
+#pragma unroll
+        for (int i = 0; i < NITER; ++i) sa[i] = sb[i] = f32x4m{0.f, 0.f, 0.f, 0.f};
+        xread(0);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            uint32_t lo[NITER], hi[NITER];
+#pragma unroll
+            for (int i = 0; i < NITER; ++i) {
+                const uint4 wv = q < 4 ? A.q0[i] : A.q1[i];
+                const uint32_t w = (q & 3) == 0 ? wv.x : (q & 3) == 1 ? wv.y : (q & 3) == 2 ? wv.z : wv.w;
+                lo[i] = opaque(w & 0x0f0f0f0fu);
+                hi[i] = opaque(w & 0xf0f0f0f0u);
+            }
+            if (q < 7) xread(q + 1);
+            if (q == 3) wread(0);
+            if (q == 7) wread(1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+#pragma unroll
+                for (int i = 0; i < NITER; ++i) {
+                    sa[i] = __builtin_amdgcn_mfma_f32_4x4x1f32(((const float*)&xa[q & 1][i])[b], (float)((lo[i] >> (8 * b)) & 0xffu), sa[i], 0, 0, 0);
+                    sb[i] = __builtin_amdgcn_mfma_f32_4x4x1f32(((const float*)&xb[q & 1][i])[b], (float)((hi[i] >> (8 * b)) & 0xffu), sb[i], 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < NITER; ++i) {
+            const int task = t + 16 * i, tk = min(task, ntask - 1);
+            const uint4 hd = A.h[i];
+            const uint32_t scw = (((hd.y >> dc.sh0) & dc.m0) | (hd.w & dc.m2)) >> dc.bsh;
+            const uint32_t mw = (((hd.z >> dc.sh0) & dc.m0) | ((hd.w >> 4) & dc.m2)) >> dc.bsh;
+            const float d = h2f(hd.x), dmin = h2f(hd.x >> 16);
+            const float dA = d * (float)(scw & 0xffu), dB16 = d * (float)((scw >> 8) & 0xffu) * 0.0625f;
+            const float mA = dmin * (float)(mw & 0xffu), mB = dmin * (float)((mw >> 8) & 0xffu);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const float2 xs = *(const float2*)(smem + (size_t)min(c, ncol - 1) * cs + (size_t)K * 4 + (size_t)tk * 8);
+                const float v = f32_pair_value(dA, sa[i][c], dB16, sb[i][c], mA, xs.x, mB, xs.y);
+                acc[c] += task < ntask ? v : 0.f;
+            }
+        }
+        wread(2);
+        // the sixteen tasks of a row lie four lanes apart: the butterfly of group_sum(acc, 16)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int off = 32; off >= 4; off >>= 1) acc[c] += __shfl_xor(acc[c], off, 64);
+        const int row = 4 * g + r;
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            if (t == c && c < ncol && row < N) y[(size_t)c * N + row] = acc[c];
+    }
+}
+
+int launch_q4k_f32m(const void* W, const float* x, float* y, int N, int K, int ncol, hipStream_t s) {
+    const size_t lds = (size_t)ncol * f32m_col_bytes(K);
+    const int grid = std::min(device_cu_count(), (N + 3) / 4);
+#define QMM_FM(IV) case IV: hipLaunchKernelGGL((k_gemv_q4k_f32m<IV>), dim3(grid), dim3(kF32mBlock), lds, s, (const uint8_t*)W, x, y, N, K, ncol); break;
+    switch ((K / 256 * 4 + 15) / 16) {
+        QMM_FM(1) QMM_FM(2) QMM_FM(3) QMM_FM(4) QMM_FM(5) QMM_FM(6)
+        default: return QMM_ERR_SHAPE;
+    }
+#undef QMM_FM
     QMM_LAUNCH_CHECK();
     return QMM_OK;
 }
@@ -1130,19 +1289,28 @@ int qmm_gemv_q4_K_f32(const void* W, const float* x, float* y, int N, int K, int
     if (ncol < 1 || ncol > 8) return QMM_ERR_SHAPE;
     (void)tpr;   // the reference's threads per row (its other values take its default, gemv.hip:1486-1489)
     hipStream_t s = (hipStream_t)stream;
-    // pair kernel: columns in launches of at most g (what fits the LDS budget); every column gets
+    // VALU pair kernel: columns in launches of at most g (what fits the LDS budget); every column gets
     // the same arithmetic whatever ncol is
     const size_t per_col = (size_t)K * 4 + (size_t)(K >> 3);
     const int g = (int)min((size_t)3, kXLdsBudget / per_col);
     if (K <= 6144 && g >= 1) {
-        for (int c0 = 0; c0 < ncol; c0 += g) {
-            const int nc = min(g, ncol - c0);
+        // Four columns at a time on the f32 matrix cores, the rest on the VALU kernel (the same bits).  Measured at
+        // 17408 x 5120, M = 4 / 6 / 8: 49 / 69 / 88 us -> 28 / 50 / 53; 1000 x 1536: M = 4 8.9 -> 5.8; 3001 x 6144: 19.7 ->
+        // 17.9.  A remainder of three takes the matrix cores where the VALU kernel is the slower one (26.8 against 36
+        // us at 17408 x 5120, 13.8 against 14.6 at 5120 x 5120; 12.6 against 12.3 at 17408 x 2048, 17.1 against 16.4 at
+        // 3001 x 6144); one or two columns cost the matrix cores as much as four.
+        for (int c0 = 0; c0 < ncol;) {
+            const int left = ncol - c0;
+            const bool mfma = left >= 4 || (left == 3 && K > 2048 && K <= 5120);
+            const int nc = mfma ? min(4, left) : min(g, left);
             const float* xc = x + (size_t)c0 * K;
             float* yc = y + (size_t)c0 * N;
-            const int e = nc == 1 ? launch_q4k_f32p<1>(W, xc, yc, N, K, s)
+            const int e = mfma    ? launch_q4k_f32m(W, xc, yc, N, K, nc, s)
+                        : nc == 1 ? launch_q4k_f32p<1>(W, xc, yc, N, K, s)
                         : nc == 2 ? launch_q4k_f32p<2>(W, xc, yc, N, K, s)
                                   : launch_q4k_f32p<3>(W, xc, yc, N, K, s);
             if (e != QMM_OK) return e;
+            c0 += nc;
         }
         return QMM_OK;
     }
