@@ -481,7 +481,9 @@ __device__ __forceinline__ void gemm_tile_core(uint4* s0, uint4* s1, uint4* s2, 
     if (it + 1 < nit) body(std::integral_constant<int, 1>(), it + 1);
     if (it + 2 < nit) body(std::integral_constant<int, 2>(), it + 2);
     __builtin_amdgcn_s_waitcnt(0);            // DMA of steps past the end
-    if constexpr (KS == 1) {
+    if constexpr (std::is_invocable_v<const Put&, gt_f32x16 (&)[NRB]>) {      // the caller takes all registers at once
+        put(acc);
+    } else if constexpr (KS == 1) {
 #pragma unroll
         for (int i = 0; i < NRB; ++i)
 #pragma unroll

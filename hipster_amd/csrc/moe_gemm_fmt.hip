@@ -1,5 +1,5 @@
-// moe_gemm_fmt.hip -- the prefill grouped expert GEMM (qmm_moe_gemm_bf16) for the expert formats other
-// than all-Q4_K, as the reference's moe_gemm takes them (engine/kernels/gemv.h:49-50,
+// moe_gemm_fmt.hip -- the prefill grouped expert GEMM on the tile core: qmm_moe_gemm_gate_up_bf16, and
+// qmm_moe_gemm_bf16 for Q4_K rows of more than two blocks and for the expert formats other than all-Q4_K, as the reference's moe_gemm takes them (engine/kernels/gemv.h:49-50,
 // gemv.hip:954-969,1377-1381: Q4_K, Q5_K, Q5_1_SOA, Q8_0_SOA, the routed and the shared expert formats
 // independent; IQ4_XS as well): over the device tile list of qmm_moe_sort,
 //   D[k0 + r][n] = sum_k A[rowtab[k0 + r]][k] * bf16(W_e[n][k])      (f32 out, sorted row order)
@@ -124,6 +124,7 @@ __device__ __forceinline__ void fmt_tile(const FArgs& a, const qmm_moe_tile tl, 
 // format, as the reference launches its routed and shared tiles apart: part 0 takes the routed
 // tiles [0, counts[0]), part 1 the shared ones [counts[0], counts[0] + counts[1]), part 2 both
 // (one format for all).  Tiles past the device count (clamped to the capacity) exit at once.
+template <int ROWS>
 __device__ __forceinline__ bool fmt_unit(const FArgs& a, int part, int* rows, qmm_moe_tile& tl, int& n0) {
     const int id = blockIdx.x, sid = id >> 3;
     const int local = 8 * (sid / a.nb) + (id & 7), nbi = sid % a.nb;
@@ -138,7 +139,7 @@ __device__ __forceinline__ bool fmt_unit(const FArgs& a, int part, int* rows, qm
         rows[threadIdx.x] = a.rowtab ? a.rowtab[k] : k;
     }
     __syncthreads();
-    n0 = nbi * FBN;
+    n0 = nbi * ROWS;
     return true;
 }
 template <int F>
@@ -147,7 +148,7 @@ __global__ void __launch_bounds__(256) k_moe_gemm_fmt(FArgs a, int part) {
     __shared__ int rows[FBM];
     qmm_moe_tile tl;
     int n0;
-    if (!fmt_unit(a, part, rows, tl, n0)) return;
+    if (!fmt_unit<FBN>(a, part, rows, tl, n0)) return;
     switch ((tl.ncols + 31) >> 5) {
         case 1: fmt_tile<1, F>(a, tl, n0, st, rows); break;
         case 2: fmt_tile<2, F>(a, tl, n0, st, rows); break;
@@ -160,21 +161,16 @@ __global__ void __launch_bounds__(256) k_moe_gemm_fmt(FArgs a, int part) {
 // output elements, straight from memory
 constexpr uint32_t kASpan = 0xf0000000u;
 template <int F>
-__device__ void moe_tile_far(const FArgs& a, const qmm_moe_tile& tl, const uint8_t* wb, size_t ldw, int n0, int nn, const int* rows) {
-    for (int i = threadIdx.x; i < tl.ncols * nn; i += blockDim.x) {
-        const int r = i / nn, n = i - r * nn;
-        const uint16_t* x = a.A + (size_t)rows[r] * a.K;
-        float acc = 0.f;
-        for (int sb = 0; sb < a.K / 32; ++sb) {
-            float w[32];
-            dq_sub32<F>(wb + (size_t)n * ldw, a.K, sb, w);
-            for (int k = 0; k < 32; ++k) acc = __builtin_fmaf(bf2f(x[32 * sb + k]), bf2f(f2bf_bits(w[k])), acc);
-        }
-        a.D[(size_t)(tl.k0 + r) * a.N + n0 + n] = acc;
+__device__ float far_dot(const uint16_t* x, const uint8_t* wrow, int K) {
+    float acc = 0.f;
+    for (int sb = 0; sb < K / 32; ++sb) {
+        float w[32];
+        dq_sub32<F>(wrow, K, sb, w);
+        for (int k = 0; k < 32; ++k) acc = __builtin_fmaf(bf2f(x[32 * sb + k]), bf2f(f2bf_bits(w[k])), acc);
     }
+    return acc;
 }
 
-// The grouped GEMM on gemm_tile.hpp's core (K % 64 == 0).  Workgroup = (tile, 32 CW weight rows).
 template <int F>
 __device__ __forceinline__ void moe_tile_unit(const FArgs& a, int part) {
     constexpr int kStage = FBM * 8;
@@ -182,7 +178,7 @@ __device__ __forceinline__ void moe_tile_unit(const FArgs& a, int part) {
     __shared__ int rows[FBM];
     qmm_moe_tile tl;
     int n0;
-    if (!fmt_unit(a, part, rows, tl, n0)) return;
+    if (!fmt_unit<FBN>(a, part, rows, tl, n0)) return;
     const int lane = threadIdx.x & 63, h = lane >> 5;
     const int n = n0 + 32 * (int)(threadIdx.x >> 6) + (lane & 31);
     const uint32_t lda = 2u * (uint32_t)a.K, ldw = (uint32_t)fmt_row_bytes_rt(F, a.K);
@@ -190,7 +186,11 @@ __device__ __forceinline__ void moe_tile_unit(const FArgs& a, int part) {
     const uint32_t wbytes = (uint32_t)min(FBN, a.N - n0) * ldw;
     const bool far = threadIdx.x < FBM && ((unsigned long long)(unsigned)rows[threadIdx.x] + 1) * lda > kASpan;
     if (__syncthreads_or(far)) {
-        moe_tile_far<F>(a, tl, wb, ldw, n0, min(FBN, a.N - n0), rows);
+        const int nn = min(FBN, a.N - n0);
+        for (int i = threadIdx.x; i < tl.ncols * nn; i += blockDim.x) {
+            const int r = i / nn, c = i - r * nn;
+            a.D[(size_t)(tl.k0 + r) * a.N + n0 + c] = far_dot<F>(a.A + (size_t)rows[r] * a.K, wb + (size_t)c * ldw, a.K);
+        }
         return;
     }
     auto go = [&](auto nrb_c) {
@@ -214,6 +214,85 @@ template <int F>
 __global__ void __launch_bounds__(256) k_moe_gemm_tile(FArgs a, int part) {
     moe_tile_unit<F>(a, part);
 }
+
+// The gate and up projections with silu (Q4_K): waves 0, 1 take 64 gate rows, waves 2, 3 the same 64 up rows and hand
+// their results over through LDS; h = bf16(silu(g) * u).  Same K order as k_moe_gemm_tile and
+// k_moe_gemm_as, so the fused and the separate calls give the same bits.  Against the 128-row, 256-column kernel
+// before it (weight blocks through LDS, one barrier-synchronised workgroup per CU; 512 experts of 512 x 2048, Zipf):
+// 96 / 512 / 2048 tokens 55 / 93 / 190 -> 40 / 82 / 174 us; 160 uniform tiles of 128 rows 123 -> 106 us.
+constexpr int kGuRows = 64;
+struct GuArgs {
+    FArgs f;                // w, wsh: gate; nb: 64-row blocks
+    const uint8_t* wu;
+    const uint8_t* wush;
+    uint16_t* H;
+};
+__device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.f + __expf(-g)) * u; }
+
+__device__ __forceinline__ void moe_gate_up_unit(const GuArgs& g) {
+    const FArgs& a = g.f;
+    constexpr int kStage = FBM * 8;
+    __shared__ uint4 s0[kStage], s1[kStage], s2[kStage], s3[kStage];
+    __shared__ int rows[FBM];
+    qmm_moe_tile tl;
+    int n0;
+    if (!fmt_unit<kGuRows>(a, 2, rows, tl, n0)) return;
+    const int lane = threadIdx.x & 63, h = lane >> 5, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool up = wave >= 2;
+    const int n = n0 + 32 * (wave & 1) + (lane & 31);
+    const uint32_t lda = 2u * (uint32_t)a.K, ldw = (uint32_t)(a.K >> 8) * 144u;
+    const size_t eo = (size_t)max(tl.expert, 0) * a.ebytes + (size_t)n0 * ldw;
+    const uint8_t* wg = (tl.expert < 0 ? a.wsh : a.w) + eo;
+    const uint8_t* wu = (tl.expert < 0 ? g.wush : g.wu) + eo;
+    const int nn = min(kGuRows, a.N - n0);
+    const bool far = threadIdx.x < FBM && ((unsigned long long)(unsigned)rows[threadIdx.x] + 1) * lda > kASpan;
+    if (__syncthreads_or(far)) {
+        for (int i = threadIdx.x; i < tl.ncols * nn; i += blockDim.x) {
+            const int r = i / nn, c = i - r * nn;
+            const uint16_t* x = a.A + (size_t)rows[r] * a.K;
+            g.H[(size_t)(tl.k0 + r) * a.N + n0 + c] = (uint16_t)f2bf_bits(
+                silu_mul(far_dot<QMM_Q4_K>(x, wg + (size_t)c * ldw, a.K), far_dot<QMM_Q4_K>(x, wu + (size_t)c * ldw, a.K)));
+        }
+        return;
+    }
+    // an up wave's rows are its base's rows 64 .. 127 (wave 2, 3 of the core's four column blocks)
+    const uint8_t* wb = up ? wu - (size_t)kGuRows * ldw : wg;
+    const uint32_t wbytes = (uint32_t)(nn + (up ? kGuRows : 0)) * ldw;
+    auto go = [&](auto nrb_c) {
+        constexpr int NRB = decltype(nrb_c)::value;
+        gemm_tile_core<QMM_Q4_K, NRB, 4, 1, 4>(
+            s0, s1, s2, s3, (const uint8_t*)a.A, kASpan, wb, wbytes, ldw, a.K,
+            [&](int r) { return r < tl.ncols ? (uint32_t)rows[r] * lda : kASpan + 0x08000000u; },
+            [&](gt_f32x16 (&acc)[NRB]) {
+                float* xch = (float*)(wave & 1 ? s1 : s0);          // the ring is no longer needed: NRB x 16 x 64 floats
+                __syncthreads();
+                if (up) {
+#pragma unroll
+                    for (int i = 0; i < NRB; ++i)
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) xch[(16 * i + e) * 64 + lane] = acc[i][e];
+                }
+                __syncthreads();
+                if (!up) {
+#pragma unroll
+                    for (int i = 0; i < NRB; ++i)
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) {
+                            const int r = 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
+                            if (r < tl.ncols && n < a.N)
+                                g.H[(size_t)(tl.k0 + r) * a.N + n] = (uint16_t)f2bf_bits(silu_mul(acc[i][e], xch[(16 * i + e) * 64 + lane]));
+                        }
+                }
+            });
+    };
+    switch ((tl.ncols + 31) >> 5) {
+        case 1: go(std::integral_constant<int, 1>()); break;
+        case 2: go(std::integral_constant<int, 2>()); break;
+        case 3: go(std::integral_constant<int, 3>()); break;
+        default: go(std::integral_constant<int, 4>()); break;
+    }
+}
+__global__ void __launch_bounds__(256) k_moe_gate_up_tile(GuArgs a) { moe_gate_up_unit(a); }
 
 int launch_fmt_part(int fmt, const FArgs& a, int part, int grid, hipStream_t s) {
     switch (fmt) {
@@ -241,6 +320,15 @@ int launch_moe_gemm_fmt(int fmt, int sfmt, const void* W, const void* Wsh, size_
     if (fmt == sfmt) return launch_fmt_part(fmt, a, 2, grid, s);
     if (int e = launch_fmt_part(fmt, a, 0, grid, s)) return e;
     return launch_fmt_part(sfmt, a, 1, grid, s);
+}
+
+int launch_moe_gate_up_tile(const void* Wg, const void* Wgsh, const void* Wu, const void* Wush, size_t ebytes, const qmm_moe_tile* tiles,
+                            const int* counts, int max_tiles, const int* rowtab, const uint16_t* A, uint16_t* H, int N, int K, hipStream_t s) {
+    GuArgs a{{(const uint8_t*)Wg, (const uint8_t*)Wgsh, ebytes, QMM_Q4_K, QMM_Q4_K, tiles, counts, max_tiles, rowtab, A, nullptr, N, K,
+              (N + kGuRows - 1) / kGuRows}, (const uint8_t*)Wu, (const uint8_t*)Wush, H};
+    hipLaunchKernelGGL(k_moe_gate_up_tile, dim3(8 * ((max_tiles + 7) / 8) * a.f.nb), dim3(256), 0, s, a);
+    QMM_LAUNCH_CHECK();
+    return QMM_OK;
 }
 
 }  // namespace qmm

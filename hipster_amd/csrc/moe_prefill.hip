@@ -293,9 +293,9 @@ __global__ void __launch_bounds__(256) k_moe_rowtok(const int* __restrict__ kpos
 // the tile, so every weight is dequantised once per workgroup, by the wave that multiplies it,
 // straight into MFMA operand registers; the two waves of a SIMD hide each other's waits.
 // v_mfma_f32_32x32x16_bf16 takes from lane l weight row l%32 and k = 8(l/32)..+7 of a 16-wide K
-// slice; for a 64-wide K step (one qs pair j of a block) these are the low nibbles of qs bytes
-// 8h..8h+7 (slice 0) and 16+8h..16+8h+7 (slice 1) and the high nibbles of the same bytes (slices
-// 2, 3), h = l/32.  A (gathered bf16 rows, DMA issued by waves 0-3) streams global -> LDS with
+// slice; which k those are is free as long as A agrees, and for a 64-wide K step (one qs pair j of a
+// block) they are the low nibbles of qs bytes 16h..16h+7 (slice 0) and 16h+8..16h+15 (slice 1) and the high
+// nibbles of the same bytes (slices 2, 3), h = l/32, as in gemm_tile.hpp.  A (gathered bf16 rows, DMA issued by waves 0-3) streams global -> LDS with
 // global_load_lds_dwordx4 through a ring of XST = 5 stages issued four steps ahead; the weight rows'
 // Q4_K blocks (144 contiguous bytes per row, so one DMA instruction covers about 7 rows: coalesced)
 // stream through a ring of block stages, DMA issued by waves 4-7: two stages (one block of 4 K steps
@@ -306,9 +306,9 @@ __global__ void __launch_bounds__(256) k_moe_rowtok(const int* __restrict__ kpos
 // chunks of 16 B, chunk c of row r in slot r*8 + (c ^ ((r >> 1) & 7)) (conflict-free fragment
 // reads); block stage: 256 rows x 144 B, row-major.  The A ring comes first in LDS, then the weight
 // ring.
-// Gate/up mode: the 256 weight rows of a workgroup are 128 gate rows (waves 0-3) and the same 128
-// up rows (waves 4-7); the up waves hand their results over through LDS and the gate waves write
-// h = bf16(silu(g) * u).
+// Rows of one Q4_K block (K = 256) run here; gate and up, and longer rows, on the tile core of gemm_tile.hpp or on
+// k_moe_gemm_as below (qmm_moe_gemm_bf16 says which and why).
+constexpr int kXMaxK = 256;
 constexpr int XBM = 128, XBW = 256, XBK = 64, XST = 5, XTHREADS = 512;
 constexpr int kXA = XBM * XBK / 8;                          // 16-byte chunks per A stage (1024)
 constexpr int kXW = 9 * XBW;                                // chunks per weight block stage (2304)
@@ -333,16 +333,14 @@ __device__ __forceinline__ void wait_steps(int rem) {
 }
 
 struct XArgs {
-    const uint8_t* w0;     // expert matrices (gate in gate/up mode), expert e at w0 + e * ebytes
+    const uint8_t* w0;     // expert matrices, expert e at w0 + e * ebytes
     const uint8_t* w0sh;   // shared-expert matrix
-    const uint8_t* w1;     // up experts (gate/up mode only)
-    const uint8_t* w1sh;
     size_t ebytes;
     const qmm_moe_tile* tiles;
     const int* counts;
     const int* rowtab;
     const uint16_t* A;
-    void* D;               // f32 [k][ldd], or bf16 h [k][ldd] in gate/up mode
+    void* D;               // f32 [k][ldd]
     int N, K, nb;          // nb = weight-row blocks per tile
     int ldd;               // row stride of D (elements)
     int cap;               // capacity of tiles (the device count is clamped to it)
@@ -363,7 +361,7 @@ __device__ __forceinline__ StepScl q4k_step_scales(const uint4 hd, int j) {
     return c;
 }
 
-template <bool GU, int NRB>
+template <int NRB>
 __device__ __forceinline__ void moe_gemm_tile(const XArgs& a, const qmm_moe_tile tl, int n0, uint4* As, const int* rows) {
     constexpr int kA = XRing<NRB>::kA, WST = XRing<NRB>::WST;
     uint4* const Ws = As + XST * kA;
@@ -372,7 +370,6 @@ __device__ __forceinline__ void moe_gemm_tile(const XArgs& a, const qmm_moe_tile
     const int K = a.K, N = a.N, nk = K / XBK, nblk = K >> 8;
     const uint32_t rowbytes = (uint32_t)(K >> 8) * 144u;
     const uint8_t* w0 = tl.expert >= 0 ? a.w0 + (size_t)tl.expert * a.ebytes : a.w0sh;
-    const uint8_t* w1 = GU ? (tl.expert >= 0 ? a.w1 + (size_t)tl.expert * a.ebytes : a.w1sh) : w0;
     const uint32_t lA = lds_addr(As), lW = lds_addr(Ws);
     // A DMA (waves 0-3): instruction q of wave wq fills slots (wq + 4q) * 64 + lane = row block q
     uint32_t aoff[NRB];
@@ -383,12 +380,12 @@ __device__ __forceinline__ void moe_gemm_tile(const XArgs& a, const qmm_moe_tile
     }
     // weight DMA (waves 4-7), one Q4_K block (144 B) of each of the 256 weight rows per 4 K steps:
     // instruction k = 9 wq + q (0..35) fills chunks 64k + lane = row (64k + lane) / 9, 16-byte part
-    // (64k + lane) % 9.  In gate/up mode instructions 0-17 are exactly the 128 gate rows.
+    // (64k + lane) % 9.  
     uint32_t woff[9];
 #pragma unroll
     for (int q = 0; q < 9; ++q) {
         const int k = 9 * wq + q, p = 64 * k + lane, row = p / 9, part = p - 9 * row;
-        woff[q] = (uint32_t)min(n0 + (GU ? (row & 127) : row), N - 1) * rowbytes + (uint32_t)(16 * part);
+        woff[q] = (uint32_t)min(n0 + row, N - 1) * rowbytes + (uint32_t)(16 * part);
     }
     auto issue = [&](int p, int st) {       // A of step p (waves 0-3)
         if (team == 0) {
@@ -404,12 +401,12 @@ __device__ __forceinline__ void moe_gemm_tile(const XArgs& a, const qmm_moe_tile
 #pragma unroll
             for (int q = 0; q < 9; ++q) {
                 const int k = 9 * wq + q;
-                dma16s((GU && k >= 18 ? w1 : w0) + b * 144, woff[q], lw + (uint32_t)(k * 1024));
+                dma16s(w0 + b * 144, woff[q], lw + (uint32_t)(k * 1024));
             }
         }
     };
     // the lane's weight row (column slot of the stage) for its MFMA column block
-    const int c0 = GU ? 128 * team + 32 * wq + fr : 32 * wave + fr;
+    const int c0 = 32 * wave + fr;
     f32x16 acc[NRB];
 #pragma unroll
     for (int i = 0; i < NRB; ++i)
@@ -419,23 +416,22 @@ __device__ __forceinline__ void moe_gemm_tile(const XArgs& a, const qmm_moe_tile
     auto afrag = [&](const uint4* la, int s, bf16x8 (&af)[NRB]) {
 #pragma unroll
         for (int i = 0; i < NRB; ++i) {
-            const uint4 v = la[(32 * i + fr) * 8 + ((2 * s + h) ^ fx)];
+            const uint4 v = la[(32 * i + fr) * 8 + ((4 * (s >> 1) + 2 * h + (s & 1)) ^ fx)];
             af[i] = *(const bf16x8*)&v;
         }
     };
     // raw weight bytes of one step for the lane's weight row, and their decode
-    struct Raw { uint4 hd; uint2 q0, q1; };
+    struct Raw { uint4 hd, q; };
     auto rawread = [&](int p, Raw& r) {     // step p: block p / 4, qs pair p % 4
         const uint8_t* rp = (const uint8_t*)(Ws + ((p >> 2) % WST) * kXW) + c0 * 144;
         const int j = p & 3;
         r.hd = *(const uint4*)rp;
-        r.q0 = *(const uint2*)(rp + 16 + 32 * j + 8 * h);
-        r.q1 = *(const uint2*)(rp + 32 + 32 * j + 8 * h);
+        r.q = *(const uint4*)(rp + 16 + 32 * j + 16 * h);
     };
     // K slice s (16 wide) of the step: s 0, 1 = low nibbles of the two qs halves (sub-block 2j),
     // s 2, 3 = their high nibbles (sub-block 2j+1)
     auto deq = [&](const Raw& r, const StepScl& c, int s) {
-        const uint2 q = (s & 1) ? r.q1 : r.q0;
+        const uint2 q = (s & 1) ? make_uint2(r.q.z, r.q.w) : make_uint2(r.q.x, r.q.y);
         return s < 2 ? q4_bf16x8_mix(q.x, q.y, 0x000f000fu, c.sa, -c.ma) : q4_bf16x8_mix(q.x, q.y, 0x00f000f0u, c.sb, -c.mb);
     };
     // before dequantising step p (waves 4-7 hold at most WST - 1 blocks in flight: block b + WST - 1
@@ -542,46 +538,19 @@ __device__ __forceinline__ void moe_gemm_tile(const XArgs& a, const qmm_moe_tile
         }
     }
     // acc[i][e] = output row 32i + 8(e/4) + 4h + e%4 of the tile, weight row n0 + (column block) + fr
-    if constexpr (GU) {
-        // up waves (4-7) hand their accumulators to the gate waves of the same SIMD through LDS
-        float* xch = (float*)As;                        // ring no longer needed: 4 x NRB x 16 x 64 floats
-        lds_barrier();
-        if (team == 1) {
+    float* D = (float*)a.D;
+    const int n = n0 + 32 * wave + fr;
 #pragma unroll
-            for (int i = 0; i < NRB; ++i)
+    for (int i = 0; i < NRB; ++i)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) xch[((wq * NRB + i) * 16 + e) * 64 + lane] = acc[i][e];
+        for (int e = 0; e < 16; ++e) {
+            const int r = 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
+            if (r < tl.ncols && n < N) D[(size_t)(tl.k0 + r) * a.ldd + n] = acc[i][e];
         }
-        lds_barrier();
-        if (team == 0) {
-            uint16_t* H = (uint16_t*)a.D;
-            const int n = n0 + 32 * wq + fr;
-#pragma unroll
-            for (int i = 0; i < NRB; ++i)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    const int r = 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
-                    if (r >= tl.ncols || n >= N) continue;
-                    const float g = acc[i][e], u = xch[((wq * NRB + i) * 16 + e) * 64 + lane];
-                    H[(size_t)(tl.k0 + r) * a.ldd + n] = (uint16_t)f2bf_bits(g / (1.f + __expf(-g)) * u);
-                }
-        }
-    } else {
-        float* D = (float*)a.D;
-        const int n = n0 + 32 * wave + fr;
-#pragma unroll
-        for (int i = 0; i < NRB; ++i)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int r = 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
-                if (r < tl.ncols && n < N) D[(size_t)(tl.k0 + r) * a.ldd + n] = acc[i][e];
-            }
-    }
 }
 
 // One workgroup per (tile, weight-row block).  Workgroup id i runs on XCD i % 8; XCD x takes tiles
 // x, x+8, x+16, ... with all their row blocks, so the blocks of one tile share its A rows in one L2.
-template <bool GU>
 __global__ void __launch_bounds__(XTHREADS) k_moe_gemm_x(XArgs a) {
     extern __shared__ __align__(16) uint8_t smem_raw[];
     __shared__ int rows[XBM];
@@ -596,19 +565,18 @@ __global__ void __launch_bounds__(XTHREADS) k_moe_gemm_x(XArgs a) {
     }
     __syncthreads();
     uint4* const As = (uint4*)smem_raw;
-    const int n0 = nbi * (GU ? XBW / 2 : XBW);
+    const int n0 = nbi * XBW;
     switch ((tl.ncols + 31) >> 5) {
-        case 1: moe_gemm_tile<GU, 1>(a, tl, n0, As, rows); break;
-        case 2: moe_gemm_tile<GU, 2>(a, tl, n0, As, rows); break;
-        case 3: moe_gemm_tile<GU, 3>(a, tl, n0, As, rows); break;
-        default: moe_gemm_tile<GU, 4>(a, tl, n0, As, rows); break;
+        case 1: moe_gemm_tile<1>(a, tl, n0, As, rows); break;
+        case 2: moe_gemm_tile<2>(a, tl, n0, As, rows); break;
+        case 3: moe_gemm_tile<3>(a, tl, n0, As, rows); break;
+        default: moe_gemm_tile<4>(a, tl, n0, As, rows); break;
     }
 }
 
-int launch_moe_gemm_x(bool gu, const XArgs& a, int max_tiles, hipStream_t s) {
+int launch_moe_gemm_x(const XArgs& a, int max_tiles, hipStream_t s) {
     const int grid = 8 * ((max_tiles + 7) / 8) * a.nb;
-    if (gu) hipLaunchKernelGGL(k_moe_gemm_x<true>, dim3(grid), dim3(XTHREADS), kXLds, s, a);
-    else hipLaunchKernelGGL(k_moe_gemm_x<false>, dim3(grid), dim3(XTHREADS), kXLds, s, a);
+    hipLaunchKernelGGL(k_moe_gemm_x, dim3(grid), dim3(XTHREADS), kXLds, s, a);
     QMM_LAUNCH_CHECK();
     return QMM_OK;
 }
@@ -621,14 +589,16 @@ int launch_moe_gemm_x(bool gu, const XArgs& a, int max_tiles, hipStream_t s) {
 // them and multiplies them against A fragments read from LDS, block after block, and stores each
 // block's f32 results.  The main loop has no workgroup barrier and no LDS writes, and A is read from
 // global memory once per unit instead of once per weight block.
-// The K order is k_moe_gemm_x's (same MFMA sequence, so the same results bit for bit): per 64-wide
-// K step lane l (weight row l%32, h = l/32) takes qs bytes 8h..8h+7 and 16+8h..16+8h+7 of the step's
-// pair, slices 0 and 1 their low nibbles, slices 2 and 3 their high nibbles, and the A fragment of
-// slice s is chunk 2s + h of the step.  A in LDS: row r at r * 1040 bytes
+// The K order is the tile core's (same MFMA sequence, so the same results bit for bit): per 64-wide
+// K step lane l (weight row l%32, h = l/32) takes qs bytes 16h..16h+15 of the step's pair in one load (as
+// two 8-byte pieces it cost the address units twice the instructions: 112 -> 106 us at 2048 tokens), slices 0
+// and 1 their low nibbles, slices 2 and 3 their high nibbles, and the A fragment of slice s is chunk
+// 4 (s / 2) + 2h + s % 2 of the step.  Two weight blocks per unit: 104.8 / 47.3 / 27.2 us at 2048 / 512 / 96 tokens
+// against 106.4 / 53.9 / 29.2 with four, whose units were too few for the CUs.  A in LDS: row r at r * 1040 bytes
 // (64 chunks of 16 B and 16 B of padding), so the 16 rows a quarter-wave reads fall in 16 distinct
 // bank groups and every fragment address is one lane base plus a constant; one DMA instruction
 // copies one row.
-constexpr int kAsK = 512, kAsThreads = 512, kAsBlocksPerUnit = 4, kAsRowBytes = 1040;
+constexpr int kAsK = 512, kAsThreads = 512, kAsBlocksPerUnit = 2, kAsRowBytes = 1040;
 constexpr bool kAsDeferStores = false;
 
 // f32 store the compiler does not see (address = wave-uniform base in SGPRs + per-lane 32-bit byte
@@ -641,9 +611,9 @@ __device__ __forceinline__ void st_f32_nc(const uint8_t* base, uint32_t voff, fl
     asm volatile("global_store_dword %0, %1, %2" : : "v"(voff), "v"(v), "s"(base) : "memory");
 }
 
-// one Q4_K block (4 K steps) of the lane's weight row: header and the lane's two 8-byte qs pieces
-// per step j (bytes 8h.. and 16+8h.. of pair j)
-struct AsRaw { uint4 hd; uint2 a0, b0, a1, b1, a2, b2, a3, b3; };
+// one Q4_K block (4 K steps) of the lane's weight row: header and the lane's 16 qs bytes per step j (bytes
+// 16h.. of pair j)
+struct AsRaw { uint4 hd, q0, q1, q2, q3; };
 
 template <int NRB>
 __device__ __forceinline__ void moe_as_unit(const XArgs& a, const qmm_moe_tile tl, int b0, int b1, const int* rows,
@@ -664,16 +634,12 @@ __device__ __forceinline__ void moe_as_unit(const XArgs& a, const qmm_moe_tile t
     auto load = [&](int g, AsRaw& r) {
         const int b = b0 + (g >> 1);
         const uint8_t* p = w + (size_t)min(b * 256 + 32 * wave + fr, N - 1) * rowbytes + (size_t)(g & 1) * 144;
-        const uint8_t* pq = p + 16 + 8 * h;
+        const uint8_t* pq = p + 16 + 16 * h;
         r.hd = ld16(p);
-        r.a0 = *(const uint2*)(pq);
-        r.b0 = *(const uint2*)(pq + 16);
-        r.a1 = *(const uint2*)(pq + 32);
-        r.b1 = *(const uint2*)(pq + 48);
-        r.a2 = *(const uint2*)(pq + 64);
-        r.b2 = *(const uint2*)(pq + 80);
-        r.a3 = *(const uint2*)(pq + 96);
-        r.b3 = *(const uint2*)(pq + 112);
+        r.q0 = ld16(pq);
+        r.q1 = ld16(pq + 32);
+        r.q2 = ld16(pq + 64);
+        r.q3 = ld16(pq + 96);
     };
     f32x16 acc0[NRB], acc1[NRB];
 #pragma unroll
@@ -684,24 +650,24 @@ __device__ __forceinline__ void moe_as_unit(const XArgs& a, const qmm_moe_tile t
     load(0, ra);
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));      // the A copy has landed (and group 0)
     __syncthreads();
-    // lane bases: row fr (row blocks 0, 1) and row 64 + fr (row blocks 2, 3), chunk h
+    // lane bases: row fr (row blocks 0, 1) and row 64 + fr (row blocks 2, 3), chunk 2h
     typedef __attribute__((address_space(3))) const uint8_t lds_u8;
-    const lds_u8* alo = (const lds_u8*)As + fr * kAsRowBytes + 16 * h;
+    const lds_u8* alo = (const lds_u8*)As + fr * kAsRowBytes + 32 * h;
     const lds_u8* ahi = alo + 64 * kAsRowBytes;
     asm volatile("" : "+v"(ahi));     // a base of its own: otherwise folded into alo + offsets past 64 KiB
 
     // K step t (0..7) of the row; the four slices' NRB MFMAs each
-    auto step = [&](const uint2 qa, const uint2 qb, const StepScl& c, int t, f32x16 (&acc)[NRB]) {
+    auto step = [&](const uint4 q, const StepScl& c, int t, f32x16 (&acc)[NRB]) {
         bf16x8 wv[4];
-        wv[0] = q4_bf16x8_mix(qa.x, qa.y, 0x000f000fu, c.sa, -c.ma);
-        wv[1] = q4_bf16x8_mix(qb.x, qb.y, 0x000f000fu, c.sa, -c.ma);
-        wv[2] = q4_bf16x8_mix(qa.x, qa.y, 0x00f000f0u, c.sb, -c.mb);
-        wv[3] = q4_bf16x8_mix(qb.x, qb.y, 0x00f000f0u, c.sb, -c.mb);
+        wv[0] = q4_bf16x8_mix(q.x, q.y, 0x000f000fu, c.sa, -c.ma);
+        wv[1] = q4_bf16x8_mix(q.z, q.w, 0x000f000fu, c.sa, -c.ma);
+        wv[2] = q4_bf16x8_mix(q.x, q.y, 0x00f000f0u, c.sb, -c.mb);
+        wv[3] = q4_bf16x8_mix(q.z, q.w, 0x00f000f0u, c.sb, -c.mb);
         // A fragments one slice ahead, each slice fenced: two slices' fragments live at most
         typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
         u32x4 af[NRB], an[NRB];
         auto rd = [&](u32x4 (&v)[NRB], int s) {
-            const int off = (8 * t + 2 * s) * 16;
+            const int off = (8 * t + 4 * (s >> 1) + (s & 1)) * 16;
 #pragma unroll
             for (int i = 0; i < NRB; ++i)
                 v[i] = *(const __attribute__((address_space(3))) u32x4*)((i < 2 ? alo : ahi) + (i & 1) * 32 * kAsRowBytes + off);
@@ -746,16 +712,16 @@ __device__ __forceinline__ void moe_as_unit(const XArgs& a, const qmm_moe_tile t
     // runs out of registers.
     auto group = [&](int g, int kb, const AsRaw& r, AsRaw& fill, f32x16 (&acc)[NRB], f32x16 (&accp)[NRB]) {
         const int t0 = 4 * kb;
-        step(r.a0, r.b0, q4k_step_scales(r.hd, 0), t0, acc);
+        step(r.q0, q4k_step_scales(r.hd, 0), t0, acc);
         __builtin_amdgcn_sched_barrier(0);
         load(min(g + 1, ng - 1), fill);
         if (kAsDeferStores && kb == 0 && g > 0) store(accp, b0 + (g >> 1) - 1);
         __builtin_amdgcn_sched_barrier(0);
-        step(r.a1, r.b1, q4k_step_scales(r.hd, 1), t0 + 1, acc);
+        step(r.q1, q4k_step_scales(r.hd, 1), t0 + 1, acc);
         __builtin_amdgcn_sched_barrier(0);
-        step(r.a2, r.b2, q4k_step_scales(r.hd, 2), t0 + 2, acc);
+        step(r.q2, q4k_step_scales(r.hd, 2), t0 + 2, acc);
         __builtin_amdgcn_sched_barrier(0);
-        step(r.a3, r.b3, q4k_step_scales(r.hd, 3), t0 + 3, acc);
+        step(r.q3, q4k_step_scales(r.hd, 3), t0 + 3, acc);
         __builtin_amdgcn_sched_barrier(0);
         if (!kAsDeferStores && kb == 1) store(acc, b0 + (g >> 1));
     };
@@ -873,13 +839,18 @@ int qmm_moe_gemm_bf16(int fmt, int shared_fmt, const void* W, const void* Wsh, s
     if (!W || !Wsh || !tiles || !counts || !A || !D) return QMM_ERR_NULL;
     if (N <= 0 || K <= 0 || K % kgran(fmt) != 0 || K % kgran(shared_fmt) != 0 || max_tiles < 0) return QMM_ERR_SHAPE;
     if (max_tiles == 0) return QMM_OK;
-    if (fmt != QMM_Q4_K || shared_fmt != QMM_Q4_K)
+    // Q4_K (2048 rows, 256 experts, top 8; this kernel against the tile core, us at 96 / 2048 / 4096 tokens): K = 256
+    // k_moe_gemm_x 17.0 / 76 / 127 against 16.4 / 85 / 145 (four K steps: the work around them decides, and its
+    // workgroups are twice as wide), K = 512 k_moe_gemm_as 20 / 88 / 153 against 21 / 110 / 196; from K = 768 on the core
+    // (30 / 142 / 233 with k_moe_gemm_x against 25 / 143 / 243, at K = 1536 49 / 250 / 391 against 48 / 228 / 381).
+    // All three take k in the same order: the same bits.
+    if (fmt != QMM_Q4_K || shared_fmt != QMM_Q4_K || (K != kAsK && K != kXMaxK))
         return launch_moe_gemm_fmt(fmt, shared_fmt, W, Wsh, ebytes, tiles, counts, max_tiles, rowtab, A, D, N, K,
                                    (hipStream_t)stream);
-    XArgs a{(const uint8_t*)W, (const uint8_t*)Wsh, nullptr, nullptr, ebytes, tiles, counts, rowtab, A, D, N, K,
+    XArgs a{(const uint8_t*)W, (const uint8_t*)Wsh, ebytes, tiles, counts, rowtab, A, D, N, K,
             (N + XBW - 1) / XBW, N, max_tiles, kAsBlocksPerUnit};
     if (K == kAsK) return launch_moe_gemm_as(a, max_tiles, (hipStream_t)stream);
-    return launch_moe_gemm_x(false, a, max_tiles, (hipStream_t)stream);
+    return launch_moe_gemm_x(a, max_tiles, (hipStream_t)stream);
 }
 
 int qmm_moe_gemm_gate_up_bf16(int fmt, int shared_fmt, const void* Wg, const void* Wgsh, const void* Wu, const void* Wush,
@@ -889,9 +860,7 @@ int qmm_moe_gemm_gate_up_bf16(int fmt, int shared_fmt, const void* Wg, const voi
     if (!Wg || !Wgsh || !Wu || !Wush || !tiles || !counts || !A || !H) return QMM_ERR_NULL;
     if (N <= 0 || K <= 0 || K % 256 != 0 || max_tiles < 0) return QMM_ERR_SHAPE;
     if (max_tiles == 0) return QMM_OK;
-    XArgs a{(const uint8_t*)Wg, (const uint8_t*)Wgsh, (const uint8_t*)Wu, (const uint8_t*)Wush, ebytes, tiles, counts,
-            rowtab, A, H, N, K, (N + XBW / 2 - 1) / (XBW / 2), N, max_tiles, 0};
-    return launch_moe_gemm_x(true, a, max_tiles, (hipStream_t)stream);
+    return launch_moe_gate_up_tile(Wg, Wgsh, Wu, Wush, ebytes, tiles, counts, max_tiles, rowtab, A, H, N, K, (hipStream_t)stream);
 }
 
 int qmm_moe_silu_bf16(const float* gate, const float* up, uint16_t* h, size_t n, void* stream) {

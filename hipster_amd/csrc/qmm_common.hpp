@@ -282,6 +282,9 @@ int gemv_fmt_dispatch_segs(int fmt, const qmm_gemv_seg* segs, int nseg, qmm_xq8 
 int launch_moe_gemm_fmt(int fmt, int sfmt, const void* W, const void* Wsh, size_t ebytes, const qmm_moe_tile* tiles,
                         const int* counts, int max_tiles, const int* rowtab, const uint16_t* A, float* D, int N, int K,
                         hipStream_t s);
+// qmm_moe_gemm_gate_up_bf16 on the tile core (moe_gemm_fmt.hip)
+int launch_moe_gate_up_tile(const void* Wg, const void* Wgsh, const void* Wu, const void* Wush, size_t ebytes, const qmm_moe_tile* tiles,
+                            const int* counts, int max_tiles, const int* rowtab, const uint16_t* A, uint16_t* H, int N, int K, hipStream_t s);
 // Q4_K GEMV of 1..16 columns over 1..4 segments sharing K on the int8 matrix cores, one launch
 // (gemv_mfma.hip); bitwise the dot4 kernels.  The dispatch of gemv.hip sends Q4_K calls of at least
 // g_mfma_min_ncol columns there.
