@@ -161,7 +161,7 @@ int moe_q8_dispatch(int fmt, const void* W, const void* Wsh, size_t ebytes, cons
 // tokens (at most 48 columns of the tile) are staged in LDS as int8 with their per-32 scales,
 // double-buffered (one barrier per block).  A sub-block is one v_mfma_i32_16x16x32_i8 per 16 tokens
 // with A = x (16 tokens x 32) and B = 32 weights x 16 rows: lane l supplies token l%16 and weight row
-// l%16, bytes k = 8(l/16)..+7 of the sub-block, and receives D[4(l/16) + r][l%16] -- four tokens of its
+// l%16, bytes k = 8 kperm(l/16)..+7 of the sub-block, and receives D[4(l/16) + r][l%16] -- four tokens of its
 // own weight row, whose sub-block scales it decoded from the block header it loaded itself.
 constexpr int kQmTok = 16, kQmMaxTok = 48, kQmRows = 64, kQmThreads = 256;
 #ifndef QMM_QM_RG
@@ -228,14 +228,25 @@ __device__ __forceinline__ void qm_x_store(QmLds& L, int buf, const QmXRegs<CB>&
     }
 }
 
-struct QmW { uint4 hd; uint2 q[4]; };
+// a lane's quants of a block: 16-byte piece kq of each couple of qs pairs (64 bytes).  As four 8-byte pieces, one a
+// pair, they were five loads a row and block instead of three, each touching 16 rows, and the address units set the
+// time (512 tokens, 16-column tiles: gate, up and down 292 -> 263 us with the activation passes between them).
+struct QmW { uint4 hd, c[2]; };
 
 __device__ __forceinline__ void qm_w_load(const uint8_t* rp, int b, int kq, QmW& w) {
     const uint8_t* blk = rp + (size_t)b * 144;
     w.hd = *(const uint4*)blk;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) w.q[j] = *(const uint2*)(blk + 16 + 32 * j + 8 * kq);
+    w.c[0] = *(const uint4*)(blk + 16 + 16 * kq);
+    w.c[1] = *(const uint4*)(blk + 80 + 16 * kq);
 }
+// a couple's pieces -> the lane's 8 bytes of each of its two pairs: one exchange between the wave's halves leaves
+// them at bytes 8 kperm(kq) of the pair, kperm = {0, 2, 1, 3}; x is read in the same order, so the dots are the same
+__device__ __forceinline__ void qm_couple(const uint4 c, uint2& a, uint2& b) {
+    const auto x = __builtin_amdgcn_permlane32_swap(c.x, c.z, false, false), y = __builtin_amdgcn_permlane32_swap(c.y, c.w, false, false);
+    a = make_uint2(x[0], y[0]);
+    b = make_uint2(x[1], y[1]);
+}
+__device__ __forceinline__ int qm_kperm(int kq) { return ((kq & 1) << 1) | (kq >> 1); }
 
 // one pass: tokens [c0, c0 + ncl) of the tile, ncl <= 16 CB, against the lane's RG weight rows (row
 // groups of 16: the x fragment of a sub-block feeds RG MFMAs)
@@ -279,7 +290,8 @@ __device__ __forceinline__ void qm_pass(const QmArgs& a, const qmm_moe_tile& tl,
             const Q4kScaleBytes sbt = q4k_scale_bytes(w[g].hd.y, w[g].hd.z, w[g].hd.w);
             scb[g] = ((uint64_t)sbt.sc_hi << 32) | sbt.sc_lo;
             mnb[g] = ((uint64_t)sbt.m_hi << 32) | sbt.m_lo;
-            q0[g] = w[g].q[0]; q1[g] = w[g].q[1]; q2[g] = w[g].q[2]; q3[g] = w[g].q[3];
+            qm_couple(w[g].c[0], q0[g], q1[g]);
+            qm_couple(w[g].c[1], q2[g], q3[g]);
         }
         // a loop, not unrolled: one qs pair (two sub-blocks) per iteration keeps the register count low
 #pragma unroll 1
@@ -297,7 +309,7 @@ __device__ __forceinline__ void qm_pass(const QmArgs& a, const qmm_moe_tile& tl,
                 }
 #pragma unroll
                 for (int cb = 0; cb < CB; ++cb) {
-                    const uint2 xv = L.x[cur][sb][kq][kQmTok * cb + tok];
+                    const uint2 xv = L.x[cur][sb][qm_kperm(kq)][kQmTok * cb + tok];
                     const long xa = (long)(((uint64_t)xv.y << 32) | (uint64_t)xv.x);
                     const float4 s01 = *(const float4*)&L.sd[cur][sb][kQmTok * cb + 4 * kq];
                     const float4 s23 = *(const float4*)&L.sd[cur][sb][kQmTok * cb + 4 * kq + 2];
