@@ -77,7 +77,7 @@ def test_gemm_wq_rows_do_not_mix(gpu):
     assert err(D[keep], ref[torch.from_numpy(keep)]) <= K ** 0.5 * 2.0 ** -24
 
 
-@pytest.mark.parametrize("fmt,N,K", [(synth.Q4_K, 130, 256), (synth.Q5_K, 128, 512), (synth.IQ4_XS, 33, 768), (synth.Q8_0_SOA, 257, 192),
+@pytest.mark.parametrize("fmt,N,K", [(synth.Q4_K, 130, 256), (synth.Q4_K, 70, 768), (synth.Q5_K, 128, 512), (synth.IQ4_XS, 33, 768), (synth.Q8_0_SOA, 257, 192),
                                      (synth.Q5_1_SOA, 2560, 640), (synth.Q5_1_SOA, 100, 96), (synth.Q8_0_SOA, 40, 64)])
 @pytest.mark.parametrize("gather", [True, False])
 def test_grouped_tiles(gpu, fmt, N, K, gather):
@@ -100,3 +100,28 @@ def test_grouped_tiles(gpu, fmt, N, K, gather):
     for e, (k0, n) in enumerate(zip(starts, sizes)):
         ref = A[idx[k0:k0 + n]].double() @ (deq(fmt, W[e]) if e < E else deq(sf, S)).t()
         assert err(D[k0:k0 + n], ref) <= K ** 0.5 * 2.0 ** -24, (e, n)
+
+
+@pytest.mark.parametrize("N,K", [(64, 256), (70, 768), (1, 512), (130, 2048)])
+def test_gate_up_tiles(gpu, N, K):
+    """the fused gate/up call at every number of row blocks and partial blocks of 64 rows: bit for bit the two
+    grouped GEMMs and silu * up it stands for"""
+    sizes = [1, 31, 32, 33, 64, 65, 97, 128]
+    E, rows = len(sizes) - 1, sum(sizes)
+    W = [dev(synth.experts(7500 + i, synth.Q4_K, E, N, K)) for i in range(2)]
+    S = [dev(synth.matrix(7502 + i, synth.Q4_K, N, K)) for i in range(2)]
+    starts = np.concatenate([[0], np.cumsum(sizes)[:-1]])
+    tiles = dev(np.array([[e, starts[e], sizes[e]] for e in range(E)] + [[-1, starts[E], sizes[E]]], np.int32))
+    counts = dev(np.array([E, 1], np.int32))
+    # weights of these blocks are of order 1e3: the activations keep gate and up in silu's range
+    A = (torch.from_numpy(synth.normal_f32(7504, (200, K))).cuda() * 1e-4).bfloat16()
+    rt = dev(synth.rng(7505).integers(0, 200, rows).astype(np.int32))
+    h, h2 = (torch.zeros((rows, N), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    eb = W[0][0].numel()
+    qmm.moe_gemm_gate_up_bf16(synth.Q4_K, synth.Q4_K, W[0], S[0], W[1], S[1], eb, tiles, counts, E + 1, rt, A, h, N, K)
+    gu = [torch.full((rows, N), float("nan"), device="cuda") for _ in range(2)]
+    for i in range(2):
+        qmm.moe_gemm_bf16(synth.Q4_K, synth.Q4_K, W[i], S[i], eb, tiles, counts, E + 1, rt, A, gu[i], N, K)
+    qmm.moe_silu_bf16(gu[0], gu[1], h2, rows * N)
+    assert torch.isfinite(h.float()).all() and h.float().abs().max() > 0
+    assert torch.equal(h.view(torch.int16), h2.view(torch.int16))
