@@ -119,6 +119,7 @@ SIGNATURES = {
     "qmm_gemm_wq": (c_int, [c_int, c_vp, c_vp, c_vp, c_int, c_int, c_int, c_vp]),
     "qmm_gemm_bf16": (c_int, [c_vp, c_vp, c_vp, c_int, c_int, c_int, c_vp]),
     "qmm_gemm_bf16_ld": (c_int, [c_vp, c_int, c_vp, c_int, c_vp, c_int, c_int, c_int, c_vp]),
+    "qmm_gemm_tile": (c_int, [c_int, c_int, c_int, c_int]),
     "qmm_f32_to_bf16": (c_int, [c_vp, c_vp, ctypes.c_size_t, c_vp]),
     "qmm_bf16_to_f32": (c_int, [c_vp, c_vp, ctypes.c_size_t, c_vp]),
     "qmm_bf16_to_f32_seg": (c_int, [c_vp, c_int, c_int, c_int, c_vp, c_int, c_vp]),

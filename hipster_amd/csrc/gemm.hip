@@ -9,8 +9,8 @@
 //   qmm_gemm_bf16           hip::BlasLt::gemm     engine/kernels/gemm.hip:125-160 (own MFMA kernel, no hipBLASLt)
 //   qmm_f32_to_bf16, qmm_bf16_to_f32, qmm_bf16_to_f32_seg, qmm_bf16_to_f32_seg2   gemm.hip:77-95
 //
-// qmm_gemm_wq and qmm_gemm_bf16 run the tile kernel of gemm_tile.hpp with the weight source as a template
-// argument; pick_tile below chooses its tile by the shape.  qmm_gemm_bf16_ld keeps a kernel without buffer
+// qmm_gemm_wq and qmm_gemm_bf16 run the kernels of gemm_tile.hpp with the weight source as a template
+// argument; pick_tile below chooses the tile by the shape.  qmm_gemm_bf16_ld keeps a kernel without buffer
 // resources (256 x 256 tiles, register-staged two-stage LDS ring) for row strides that no resource spans.
 #include "fmt_dequant.hpp"
 #include "gemm_tile.hpp"
@@ -260,64 +260,97 @@ __global__ void __launch_bounds__(256) k_gemm(const uint16_t* __restrict__ A, co
     }
 }
 // ------------------------------------------------------------------------------------------
-// Tile choice of the dequantising GEMM (gemm_tile.hpp).  A workgroup fills a CU, so a shape takes
-// ceil(tiles / CUs) rounds of about K / 64 / KS steps each, and the choice is the tile with the least
-// rounds x (steps x step time + launch and reduction).  Step times in 0.01 us, measured with Q4_K weights on
-// 256 CUs: large tiles do the most work per step (192 x 256: 34 blocks of 32 x 32 x 64 per us, 32 x 32 with
-// eight K groups: 9) and small ones fill the chip where M x N is small.  The choice does not look at the
-// format, so every weight source gets the same K order.
-struct TileShape { int nrb, cw, ks, step, fixed; };
-constexpr TileShape kTiles[] = {{1, 1, 8, 75, 200}, {2, 1, 8, 110, 250}, {2, 2, 4, 75, 200}, {4, 2, 4, 120, 300}, {4, 4, 2, 105, 300},
-                                {4, 8, 1, 90, 400}, {5, 8, 1, 108, 400}, {6, 8, 1, 129, 400}, {8, 8, 1, 150, 400}};
+// Tile choice of the dequantising GEMM (gemm_tile.hpp).  Every tile runs the same chain of matrix instructions over K, so the
+// choice changes no bit: it may look at everything.  The busiest of the CUs gets q = ceil(tiles / CUs) workgroups, and a
+// step of 64 takes it about kStep[format][tile].first ns for one of them and .more for each further one (measured on 256
+// CUs with 256 q tiles, q = 1 .. 3, K = 2048 and 8192; two or three workgroups of the small tiles share a CU and hide
+// each other's waits).  The large tiles do the most work per ns (192 x 256: 37 blocks of 32 x 32 per us, 16 x 16 by
+// producers: 3 to 10), the small ones fill the chip where M x N is small: 40 x 1024 x 5120 in 9 us against 38 with
+// 64 x 128, 2048 x 17408 x 5120 in 316 us against 1050 with 64 x 64 by producers.
+struct TileShape { int bm, bn, fixed, more; };       // rows, columns; ns for the launch, first loads and stores, the same for each further workgroup
+constexpr TileShape kTiles[] = {{16, 16, 4000, 0},      {32, 16, 3200, 1400},   {64, 16, 3400, 2400},   {48, 32, 4500, 1500},   {64, 32, 4700, 1600},
+                                {64, 64, 2600, 900},    {128, 64, 4500, 1800},  {64, 128, 2500, 3800},  {96, 128, 6100, 1800},  {128, 128, 7900, 1800},
+                                {160, 128, 8100, 2100}, {128, 256, 8500, 4800}, {192, 256, 10900, 8000}, {256, 256, 13200, 9200}};
 constexpr int kNumTiles = (int)(sizeof(kTiles) / sizeof(kTiles[0]));
+struct StepNs { uint16_t first, more; };
+constexpr StepNs kStep[7][kNumTiles] = {
+    {{77, 74}, {104, 104}, {137, 131}, {161, 207}, {178, 228}, {360, 357}, {429, 430}, {463, 318}, {496, 398}, {540, 484}, {630, 573}, {931, 944}, {1278, 1243}, {1644, 1628}},   // Q4_K
+    {{103, 99}, {126, 130}, {161, 177}, {207, 243}, {226, 284}, {452, 441}, {523, 508}, {525, 369}, {537, 489}, {662, 545}, {716, 637}, {1090, 1145}, {1405, 1389}, {1726, 1695}},   // Q5_K
+    {{99, 75}, {125, 128}, {163, 159}, {185, 210}, {204, 231}, {336, 330}, {421, 411}, {555, 445}, {627, 485}, {711, 587}, {756, 668}, {1143, 1210}, {1453, 1461}, {1768, 1772}},   // IQ4_XS
+    {{141, 40}, {148, 119}, {172, 175}, {164, 204}, {177, 216}, {361, 347}, {423, 413}, {628, 460}, {704, 505}, {752, 582}, {802, 657}, {1173, 1207}, {1468, 1498}, {1810, 1747}},   // Q6_K
+    {{87, 90}, {112, 141}, {147, 181}, {211, 207}, {232, 226}, {390, 372}, {464, 440}, {550, 474}, {607, 517}, {642, 594}, {684, 676}, {1096, 1131}, {1382, 1399}, {1672, 1674}},   // Q8_0
+    {{109, 87}, {130, 143}, {166, 175}, {191, 239}, {210, 255}, {395, 371}, {462, 453}, {608, 439}, {686, 525}, {776, 578}, {813, 671}, {1236, 1234}, {1472, 1515}, {1780, 1755}},   // Q5_1
+    {{74, 88}, {103, 113}, {166, 168}, {202, 185}, {224, 211}, {352, 339}, {442, 442}, {612, 591}, {666, 664}, {727, 736}, {815, 824}, {1336, 1223}, {1521, 1537}, {1732, 1727}},   // bf16
+};
+constexpr int step_row(int f) { return f == QMM_W_BF16 ? 6 : f; }
+static_assert(QMM_Q4_K == 0 && QMM_Q5_K == 1 && QMM_IQ4_XS == 2 && QMM_Q6_K_SOA == 3 && QMM_Q8_0_SOA == 4 && QMM_Q5_1_SOA == 5, "");
 
-int tile_count(const TileShape& t, int M, int N) {
-    return ((M + 32 * t.nrb - 1) / (32 * t.nrb)) * ((N + 32 * t.cw - 1) / (32 * t.cw));
-}
+int tile_count(const TileShape& t, int M, int N) { return ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn); }
 
 // the operands' span in a tile must fit a buffer resource (32-bit offsets)
 bool tile_fits(const TileShape& t, const GemmArgs& a) {
-    const size_t ra = (size_t)std::min(a.M, 32 * t.nrb) - 1, rw = (size_t)std::min(a.N, 32 * t.cw) - 1;
+    const size_t ra = (size_t)std::min(a.M, t.bm) - 1, rw = (size_t)std::min(a.N, t.bn) - 1;
     return ra * a.lda + (size_t)a.K * 2 <= 0xffffffffu && rw * a.ldw + a.rowbytes <= 0xffffffffu;
 }
 
-int pick_tile(const GemmArgs& a) {
+int pick_tile(int f, const GemmArgs& a) {
     int best = -1;
     long long cost = 0;
     const int cus = device_cu_count(), nk = a.K / 64;
     for (int i = 0; i < kNumTiles; ++i) {
         const TileShape& t = kTiles[i];
         if (!tile_fits(t, a)) continue;
-        const long long rounds = (tile_count(t, a.M, a.N) + cus - 1) / cus;
-        const long long c = rounds * ((long long)gt_local_steps(nk, t.ks) * t.step + t.fixed);
+        const StepNs& st = kStep[step_row(f)][i];
+        const long long q = (tile_count(t, a.M, a.N) + cus - 1) / cus;
+        const long long c = nk * (st.first + (q - 1) * st.more) + t.fixed + (q - 1) * t.more;
         if (best < 0 || c < cost) { best = i; cost = c; }
     }
     return best;
 }
 
-template <int F, bool OUT_BF16, int NRB, int CW, int KS, int ST>
+template <int F, bool OUT_BF16, int NRB, int CW>
 int launch_tile(const GemmArgs& a, hipStream_t s) {
-    const int grid = tile_count(TileShape{NRB, CW, KS, 0, 0}, a.M, a.N);
-    hipLaunchKernelGGL((k_gemm_tile<F, NRB, CW, KS, ST, OUT_BF16>), dim3(grid), dim3(64 * CW * KS), 0, s, a);
+    hipLaunchKernelGGL((k_gemm_tile<F, NRB, CW, OUT_BF16>), dim3(tile_count({32 * NRB, 32 * CW, 0, 0}, a.M, a.N)), dim3(64 * CW), 0, s, a);
+    QMM_LAUNCH_CHECK();
+    return QMM_OK;
+}
+template <int F, bool OUT_BF16, int R, int CB, int CR, int CC, int B>
+int launch_few(const GemmArgs& a, hipStream_t s) {
+    hipLaunchKernelGGL((k_gemm_few<F, R, CB, CR, CC, B, OUT_BF16>), dim3(tile_count({16 * R, 16 * CB, 0, 0}, a.M, a.N)),
+                       dim3(64 * gf_waves<F, R, CB, CR, CC, B>), 0, s, a);
     QMM_LAUNCH_CHECK();
     return QMM_OK;
 }
 
 // D = A . W^T with W from source F, f32 or bf16 (RNE) out; K % 64 == 0
 template <int F, bool OUT_BF16>
-int launch_gemm(const GemmArgs& a, hipStream_t s) {
-    switch (pick_tile(a)) {
-        case 0: return launch_tile<F, OUT_BF16, 1, 1, 8, 4>(a, s);
-        case 1: return launch_tile<F, OUT_BF16, 2, 1, 8, 2>(a, s);
-        case 2: return launch_tile<F, OUT_BF16, 2, 2, 4, 4>(a, s);
-        case 3: return launch_tile<F, OUT_BF16, 4, 2, 4, 2>(a, s);
-        case 4: return launch_tile<F, OUT_BF16, 4, 4, 2, 4>(a, s);
-        case 5: return launch_tile<F, OUT_BF16, 4, 8, 1, 4>(a, s);
-        case 6: return launch_tile<F, OUT_BF16, 5, 8, 1, 4>(a, s);
-        case 7: return launch_tile<F, OUT_BF16, 6, 8, 1, 4>(a, s);
-        // bf16 rows: four steps' weights (64 registers) beside 128 accumulators would spill
-        case 8: return launch_tile<F, OUT_BF16, 8, 8, 1, F == QMM_W_BF16 ? 2 : 4>(a, s);
-        default: return QMM_ERR_SHAPE;
+int launch_gemm(GemmArgs a, hipStream_t s) {
+    const int tile = pick_tile(F, a);
+    if (tile < 0) return QMM_ERR_SHAPE;
+    // rows past M and N read at an offset that is out of the tile's range (and stays so with a row's bytes added), or at
+    // row 0 where the range leaves no such offset
+    const TileShape& t = kTiles[tile];
+    auto past = [](size_t rows, size_t ld, size_t row) {
+        const size_t span = (rows - 1) * ld + row;
+        return span + row <= 0xffffff00u ? (uint32_t)(0xffffff00u - row) : 0u;
+    };
+    a.apast = past((size_t)std::min(a.M, t.bm), a.lda, (size_t)a.K * 2);
+    a.wpast = past((size_t)std::min(a.N, t.bn), a.ldw, a.rowbytes);
+    switch (tile) {
+        case 0: return launch_few<F, OUT_BF16, 1, 1, 1, 1, 4>(a, s);
+        case 1: return launch_few<F, OUT_BF16, 2, 1, 2, 1, 4>(a, s);
+        case 2: return launch_few<F, OUT_BF16, 4, 1, 2, 1, 4>(a, s);
+        case 3: return launch_few<F, OUT_BF16, 3, 2, 3, 1, 4>(a, s);
+        case 4: return launch_few<F, OUT_BF16, 4, 2, 2, 2, 4>(a, s);
+        case 5: return launch_few<F, OUT_BF16, 4, 4, 2, 2, 2>(a, s);
+        case 6: return launch_few<F, OUT_BF16, 8, 4, 4, 2, 2>(a, s);
+        case 7: return launch_tile<F, OUT_BF16, 2, 4>(a, s);
+        case 8: return launch_tile<F, OUT_BF16, 3, 4>(a, s);
+        case 9: return launch_tile<F, OUT_BF16, 4, 4>(a, s);
+        case 10: return launch_tile<F, OUT_BF16, 5, 4>(a, s);
+        case 11: return launch_tile<F, OUT_BF16, 4, 8>(a, s);
+        case 12: return launch_tile<F, OUT_BF16, 6, 8>(a, s);
+        default: return launch_tile<F, OUT_BF16, 8, 8>(a, s);
     }
 }
 
@@ -393,7 +426,7 @@ int qmm_gemm_wq(int fmt, const void* W, const uint16_t* A, float* D, int M, int 
     const int kg = (fmt == QMM_Q8_0_SOA || fmt == QMM_Q5_1_SOA) ? 2 * GBK : fmt == QMM_Q6_K_SOA ? 512 : 256;
     if (M <= 0 || N <= 0 || K <= 0 || K % kg != 0) return QMM_ERR_SHAPE;
     const size_t rb = fmt_row_bytes_rt(fmt, K);
-    const GemmArgs a{(const uint8_t*)A, (const uint8_t*)W, D, (uint32_t)K * 2u, (uint32_t)rb, (uint32_t)rb, M, N, K, N};
+    const GemmArgs a{(const uint8_t*)A, (const uint8_t*)W, D, (uint32_t)K * 2u, (uint32_t)rb, (uint32_t)rb, M, N, K, N, 0, 0};
     hipStream_t s = (hipStream_t)stream;
     switch (fmt) {
         case QMM_Q4_K: return launch_gemm<QMM_Q4_K, false>(a, s);
@@ -412,14 +445,21 @@ int qmm_gemm_bf16_ld(const uint16_t* A, int lda, const uint16_t* W, int ldw, uin
     if (((uintptr_t)A | (uintptr_t)W) % 16 != 0 || lda % 8 != 0 || ldw % 8 != 0) return QMM_ERR_ARG;
     // the DMA of A addresses rows with 32-bit element offsets
     if ((uint64_t)(M - 1) * (uint64_t)lda + (uint64_t)K > 0xffffffffull) return QMM_ERR_SHAPE;
-    const GemmArgs a{(const uint8_t*)A, (const uint8_t*)W, D, (uint32_t)lda * 2u, (uint32_t)ldw * 2u, (uint32_t)K * 2u, M, N, K, N};
-    if (pick_tile(a) >= 0) return launch_gemm<QMM_W_BF16, true>(a, (hipStream_t)stream);
+    const GemmArgs a{(const uint8_t*)A, (const uint8_t*)W, D, (uint32_t)lda * 2u, (uint32_t)ldw * 2u, (uint32_t)K * 2u, M, N, K, N, 0, 0};
+    if (pick_tile(QMM_W_BF16, a) >= 0) return launch_gemm<QMM_W_BF16, true>(a, (hipStream_t)stream);
     // rows so far apart that no tile's span fits a buffer resource
     const int grid = ((M + GBM - 1) / GBM) * ((N + GBN - 1) / GBN);
     hipLaunchKernelGGL((k_gemm<BLoadBf16, uint16_t, true>), dim3(grid), dim3(256), kGemmLds, (hipStream_t)stream, A, W, (void*)D, M, N,
                        K, lda, ldw);
     QMM_LAUNCH_CHECK();
     return QMM_OK;
+}
+
+int qmm_gemm_tile(int fmt, int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0 || fmt == QMM_Q6_K || fmt > QMM_Q5_1_SOA) return QMM_ERR_ARG;
+    const int f = fmt < 0 ? QMM_W_BF16 : fmt;
+    const uint32_t rb = fmt < 0 ? (uint32_t)K * 2u : (uint32_t)fmt_row_bytes_rt(fmt, K);
+    return pick_tile(f, GemmArgs{nullptr, nullptr, nullptr, (uint32_t)K * 2u, rb, rb, M, N, K, N, 0, 0});
 }
 
 int qmm_gemm_bf16(const uint16_t* A, const uint16_t* W, uint16_t* D, int M, int N, int K, void* stream) {

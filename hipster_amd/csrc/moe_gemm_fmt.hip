@@ -6,8 +6,7 @@
 // with W_e dequantised exactly (the arithmetic of qmm_dequant_bf16) and bf16 MFMA, f32 accumulation.
 //
 // Workgroup = (tile, 128 weight rows), 256 threads = 4 waves, the core of gemm_tile.hpp with the tile's
-// ceil(rows / 32) row blocks.  One K group and four stages: of the shapes measured (128 or 256 columns, 1, 2 or 4 K
-// groups, two or four stages) the best at 64, 600 and 2048 tokens.  Weights are read once a tile; with the 32-k
+// ceil(rows / 32) row blocks: 128 columns were better than 256 at 64, 600 and 2048 tokens.  Weights are read once a tile; with the 32-k
 // steps through LDS of k_moe_gemm_fmt before it, waiting for its loads at every step, the calls took
 // (512 experts, Zipf routing, HIP graph replay, gate Q5_K 640 x 2560 / down Q5_1 2560 x 640):
 //   64 tokens 134 / 78 -> 37 / 35 us,  600 tokens 225 / 207 -> 82 / 107 us,  2048 tokens 368 / 366 -> 153 / 212 us
@@ -195,8 +194,8 @@ __device__ __forceinline__ void moe_tile_unit(const FArgs& a, int part) {
     }
     auto go = [&](auto nrb_c) {
         constexpr int NRB = decltype(nrb_c)::value;
-        gemm_tile_core<F, NRB, FBN / 32, 1, 4>(
-            s0, s1, s2, s3, (const uint8_t*)a.A, kASpan, wb, wbytes, ldw, a.K,
+        gemm_tile_core<F, NRB, FBN / 32>(
+            s0, s1, s2, s3, (const uint8_t*)a.A, kASpan, wb, wbytes, (uint32_t)(n - n0) * ldw, a.K,
             [&](int r) { return r < tl.ncols ? (uint32_t)rows[r] * lda : kASpan + 0x08000000u; },   // past the span: zeros
             [&](int i, int e, float v) {
                 const int r = 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
@@ -260,8 +259,8 @@ __device__ __forceinline__ void moe_gate_up_unit(const GuArgs& g) {
     const uint32_t wbytes = (uint32_t)(nn + (up ? kGuRows : 0)) * ldw;
     auto go = [&](auto nrb_c) {
         constexpr int NRB = decltype(nrb_c)::value;
-        gemm_tile_core<QMM_Q4_K, NRB, 4, 1, 4>(
-            s0, s1, s2, s3, (const uint8_t*)a.A, kASpan, wb, wbytes, ldw, a.K,
+        gemm_tile_core<QMM_Q4_K, NRB, 4>(
+            s0, s1, s2, s3, (const uint8_t*)a.A, kASpan, wb, wbytes, (uint32_t)(32 * wave + (lane & 31)) * ldw, a.K,
             [&](int r) { return r < tl.ncols ? (uint32_t)rows[r] * lda : kASpan + 0x08000000u; },
             [&](gt_f32x16 (&acc)[NRB]) {
                 float* xch = (float*)(wave & 1 ? s1 : s0);          // the ring is no longer needed: NRB x 16 x 64 floats

@@ -322,6 +322,11 @@ def gemm_bf16_ld(A, lda, W, ldw, D, M, N, K, stream=None):
     check(_lib.lib().qmm_gemm_bf16_ld(_p(A), lda, _p(W), ldw, _p(D), M, N, K, _stream(stream)), "gemm_bf16_ld")
 
 
+def gemm_tile(fmt, M, N, K):
+    """Index of the tile that gemm_wq (fmt < 0: gemm_bf16) runs for this shape."""
+    return _lib.lib().qmm_gemm_tile(fmt, M, N, K)
+
+
 def f32_to_bf16(x, out, n, stream=None):
     check(_lib.lib().qmm_f32_to_bf16(_p(x), _p(out), n, _stream(stream)), "f32_to_bf16")
 

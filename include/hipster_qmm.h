@@ -307,16 +307,21 @@ int qmm_dequant_bf16(int fmt, const void* W, uint16_t* out, int N, int K, void* 
  * pair (engine/src/qwen35.cpp:204-239, engine/src/qwen4exp.cpp:513-527) with one launch and no
  * scratch.  fmt: Q4_K, Q5_K, IQ4_XS (K % 256), Q6_K_SOA (K % 512), Q8_0_SOA, Q5_1_SOA (K % 128);
  * GGUF-native Q6_K rows take qmm_dequant_bf16 + qmm_gemm_bf16 (the engine repacks Q6_K to the SoA
- * layout at load). */
+ * layout at load).  An output element is one chain of matrix instructions over K, the same for every M,
+ * N, format and device: a prompt cut into other chunks or a matrix joined to another gives the same bits,
+ * and rounded to bf16 they are qmm_gemm_bf16's on the dequantised rows. */
 int qmm_gemm_wq(int fmt, const void* W, const uint16_t* A, float* D, int M, int N, int K, void* stream);
 /* D[M][N] bf16 = A[M][K] bf16 . W[N][K]^T bf16, f32 accumulate, RNE to bf16 (reference: BlasLt::gemm,
  * gemm.h:27, gemm.hip:125-160; here an own MFMA kernel, no hipBLASLt: the fused GEMM's kernel with bf16
- * rows as its weight source when K % 128 == 0).  K % 64 == 0. */
+ * rows as its weight source).  K % 64 == 0. */
 int qmm_gemm_bf16(const uint16_t* A, const uint16_t* W, uint16_t* D, int M, int N, int K, void* stream);
 /* the same with row strides (elements) for A and W (reference: BlasLt::gemm_ld, gemm.h:29,
  * gemm.hip:125-160; the split-K halves of qwen35.cpp:230-231): A[m][k] at A[m*lda + k], W[n][k] at
  * W[n*ldw + k]; D [M][N] dense.  lda, ldw >= K and multiples of 8, A and W 16-byte aligned. */
 int qmm_gemm_bf16_ld(const uint16_t* A, int lda, const uint16_t* W, int ldw, uint16_t* D, int M, int N, int K, void* stream);
+/* the tile (0 ..) that a GEMM of this shape runs, fmt < 0: bf16 rows; for tests and benchmarks (the choice
+ * changes no bit) */
+int qmm_gemm_tile(int fmt, int M, int N, int K);
 /* bf16 helpers (reference: gemm.h:14-20, gemm.hip:77-95) */
 int qmm_f32_to_bf16(const float* x, uint16_t* out, size_t n, void* stream);
 int qmm_bf16_to_f32(const uint16_t* x, float* out, size_t n, void* stream);

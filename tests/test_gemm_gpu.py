@@ -84,8 +84,7 @@ def test_gemm_wq_small_and_ragged(gpu, M, N, K):
 
 @pytest.mark.parametrize("M,N,K", [(2048, 8548, 512), (300, 40000, 256)])
 def test_gemm_wq_split_last_round(gpu, M, N, K):
-    """shapes whose last round of 256 x 256 tiles would be thin: the trailing columns (ragged) go to
-    the grouped kernel's implicit row tiles (ragged M too); the whole D is checked"""
+    """many columns against few K steps, ragged on both sides; the whole D is checked"""
     gemm_check(M, N, K, 1350 + M, npairs=64)
 
 
@@ -95,8 +94,7 @@ def test_gemm_wq_config3_full_shape(gpu):
 
 @pytest.mark.parametrize("M,N,K", [(256, 128, 64), (300, 515, 640), (2048, 2048, 2048), (129, 384, 192)])
 def test_gemm_bf16(gpu, M, N, K):
-    """K % 128 == 0 runs the two-waves-per-SIMD kernel with bf16 rows as its W source, other K the
-    4-wave kernel"""
+    """bf16 rows as the weight source, K in whole rounds of the ring's stages and not"""
     A = synth.to_bf16_bits(synth.normal_f32(70 + M, (M, K)))
     W = synth.to_bf16_bits(synth.normal_f32(71 + N, (N, K)))
     D = torch.zeros((M, N), dtype=torch.bfloat16, device="cuda")
@@ -129,8 +127,7 @@ def test_gemm_wq_other_formats(gpu, fmt, M, N, K):
 @pytest.mark.parametrize("M,N,K", [(512, 512, 1024), (300, 768, 2048)])
 def test_gemm_wq_q4k_is_the_bf16_gemm_of_its_dequantisation(gpu, M, N, K):
     """the fused Q4_K GEMM feeds the matrix cores exactly qmm_dequant_bf16's weights: rounded to bf16 its
-    f32 output equals, bit for bit, the bf16 GEMM (the same kernel body and K order) on the dequantised
-    rows"""
+    f32 output equals, bit for bit, the bf16 GEMM (the same chain over K) on the dequantised rows"""
     W = dev(synth.matrix(1460 + N, synth.Q4_K, N, K))
     A = bf16_dev(synth.to_bf16_bits(synth.normal_f32(1461 + M, (M, K))))
     D = torch.full((M, N), float("nan"), device="cuda")

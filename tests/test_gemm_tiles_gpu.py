@@ -1,10 +1,11 @@
-"""The tile kernel of the prefill GEMMs (gemm_tile.hpp) where its tilings can go wrong: every weight
-source, sizes around the edges of each tile (rows 32, 64, 128, 192; columns 32, 64, 128, 256), K steps that do not
-divide among the K groups, one row, one column, and a shape per tile choice.
+"""The kernels of the prefill GEMMs (gemm_tile.hpp) where their tilings can go wrong: every weight source, sizes
+around the edges of each tile (rows 16 .. 256, columns 16 .. 256), K steps that do not divide among the ring's stages, one
+row, one column, and every tile of the choice (test_every_tile_is_run asks the library which one a shape takes).
 
-Bound: every product of two bf16 values is exact in f32, so only the K additions round.  Their errors add
-up as a random walk, each at most 2^-24 of a partial sum that grows like sqrt(k): sqrt(K) 2^-24 relative
-in the 2-norm, against the float64 product of the same bf16 operands."""
+Bound: every product of two bf16 values is exact in f32, so only the K additions round, each by at most 2^-24
+of a partial sum, which is at most |a| |w| (Cauchy-Schwarz).  Their errors add up as a random walk: an element is
+within 4 sqrt(K) 2^-24 |a| |w| of the float64 product of the same bf16 operands (over six standard deviations of it), and a
+matrix within sqrt(K) 2^-24 in the relative 2-norm."""
 import numpy as np
 import pytest
 import torch
@@ -12,9 +13,14 @@ import torch
 from hipster_amd import qmm, synth
 from tests.gpu_util import dev
 
-pytestmark = pytest.mark.gpu
+GPU = pytest.mark.gpu
 SHAPES = [(1, 70, 512), (70, 1, 512), (17, 33, 1536), (33, 1024, 2560), (40, 6144, 1024), (65, 63, 512), (129, 257, 1024), (300, 2500, 512),
           (193, 8200, 512), (385, 17000, 512), (1100, 300, 1536), (2048, 5120, 512)]
+# a shape of every tile, ragged on both sides, two or more rounds of the ring's stages
+TILES = [(1, 4099, 1024), (17, 2560, 1536), (2077, 49, 1024), (17, 4147, 1024), (50, 4121, 1536), (100, 5100, 1024), (2311, 775, 512),
+         (17, 16439, 512), (67, 17287, 512), (100, 16577, 1536), (259, 13135, 512), (294, 16537, 512), (485, 16487, 512), (774, 14659, 512)]
+FORMATS = [synth.Q4_K, synth.Q5_K, synth.IQ4_XS, synth.Q6_K_SOA, synth.Q8_0_SOA, synth.Q5_1_SOA]
+BF16 = -1
 
 
 def operands(fmt, M, N, K, seed):
@@ -30,29 +36,68 @@ def err(got, ref):
     return ((got.double() - ref).norm() / ref.norm()).item()
 
 
-@pytest.mark.parametrize("fmt", [synth.Q4_K, synth.Q5_K, synth.IQ4_XS, synth.Q6_K_SOA, synth.Q8_0_SOA, synth.Q5_1_SOA])
-@pytest.mark.parametrize("M,N,K", SHAPES)
+def check(D, A, Wb, ref, K):
+    """every element within its bound, and written"""
+    bound = 4 * K ** 0.5 * 2.0 ** -24 * A.double().norm(dim=1)[:, None] * Wb.double().norm(dim=1)[None, :]
+    assert ((D.double() - ref).abs() <= bound).all()
+    assert err(D, ref) <= K ** 0.5 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("M,N,K", SHAPES + TILES)
+@GPU
 def test_gemm_wq_tiles(gpu, fmt, M, N, K):
     A, W, Wb, ref = operands(fmt, M, N, K, 7000 + M + N)
     D = torch.full((M, N), float("nan"), device="cuda")
     qmm.gemm_wq(fmt, W, A, D, M, N, K)
-    assert err(D, ref) <= K ** 0.5 * 2.0 ** -24
-    # the bf16 GEMM takes the same tile and K order, but lanes of some formats hold k in another order: the same
-    # sums within the bound, then one rounding to bf16 (8 bits: 2^-8 at most)
-    Db = torch.zeros((M, N), dtype=torch.bfloat16, device="cuda")
+    check(D, A, Wb, ref, K)
+    # the bf16 GEMM on the dequantised rows is the same chain, rounded once more
+    Db = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
     qmm.gemm_bf16(A, Wb, Db, M, N, K)
-    assert err(Db, ref) <= 2.0 ** -8
+    assert torch.equal(Db.view(torch.int16), D.bfloat16().view(torch.int16))
+
+
+@pytest.mark.parametrize("fmt", FORMATS + [BF16])
+def test_every_tile_is_run(fmt):
+    assert sorted({qmm.gemm_tile(fmt, *s) for s in SHAPES + TILES}) == list(range(14))
+
+
+@pytest.mark.parametrize("fmt,N,K", [(f, n, k) for f in FORMATS for n, k in ((700, 1536), (16500, 512))] +
+                         [(synth.Q8_0_SOA, 260, 640), (synth.Q5_1_SOA, 260, 384)])
+@GPU
+def test_bits_do_not_depend_on_rows_or_columns_of_the_call(gpu, fmt, N, K):
+    """the rows of a prompt in chunks of any size, and the columns of a matrix apart or joined: the bits of one call"""
+    M = 1600
+    A, W, Wb, _ = operands(fmt, M, N, K, 7600 + N)
+    full = torch.full((M, N), float("nan"), device="cuda")
+    qmm.gemm_wq(fmt, W, A, full, M, N, K)
+    tiles = {qmm.gemm_tile(fmt, M, N, K)}
+    m0 = 0
+    for m in (1, 16, 17, 40, 64, 100, 129, 200, 300, 733):
+        D = torch.full((m, N), float("nan"), device="cuda")
+        qmm.gemm_wq(fmt, W, A[m0:m0 + m], D, m, N, K)
+        assert torch.equal(D.view(torch.int32), full[m0:m0 + m].view(torch.int32)), (m, qmm.gemm_tile(fmt, m, N, K))
+        tiles.add(qmm.gemm_tile(fmt, m, N, K))
+        m0 += m
+    assert m0 == M and len(tiles) >= 3, tiles
+    for n0, n in ((0, 3), (3, 100), (103, N - 103)):
+        for m in (16, 300):
+            D = torch.full((m, n), float("nan"), device="cuda")
+            qmm.gemm_wq(fmt, W[n0:n0 + n], A[:m], D, m, n, K)
+            assert torch.equal(D.view(torch.int32), full[:m, n0:n0 + n].contiguous().view(torch.int32)), (n, m)
 
 
 @pytest.mark.parametrize("fmt,K", [(synth.Q8_0_SOA, 128), (synth.Q5_1_SOA, 640), (synth.Q4_K, 256), (synth.Q6_K_SOA, 512)])
+@GPU
 def test_gemm_wq_short_k(gpu, fmt, K):
-    """fewer K steps than K groups, and a last group without a step"""
+    """fewer K steps than the ring has stages, and a last round that is not full"""
     A, W, Wb, ref = operands(fmt, 21, 70, K, 7100 + K)
     D = torch.full((21, 70), float("nan"), device="cuda")
     qmm.gemm_wq(fmt, W, A, D, 21, 70, K)
     assert err(D, ref) <= K ** 0.5 * 2.0 ** -24
 
 
+@GPU
 def test_gemm_bf16_odd_step_count_and_strides(gpu):
     """K = 192 (three steps) and operands that are views of wider matrices, garbage (NaN) around them"""
     M, N, K = 45, 300, 192
@@ -60,11 +105,15 @@ def test_gemm_bf16_odd_step_count_and_strides(gpu):
     W = torch.full((N, 200), float("nan"), device="cuda", dtype=torch.bfloat16)
     A[:, :K] = torch.from_numpy(synth.normal_f32(7200, (M, K))).cuda().bfloat16()
     W[:, :K] = torch.from_numpy(synth.normal_f32(7201, (N, K))).cuda().bfloat16()
-    D = torch.zeros((M, N), dtype=torch.bfloat16, device="cuda")
+    D = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
     qmm.gemm_bf16_ld(A, 256, W, 200, D, M, N, K)
-    assert err(D, A[:, :K].double() @ W[:, :K].double().t()) <= 2.0 ** -8
+    a, w = A[:, :K].double(), W[:, :K].double()
+    ref = a @ w.t()
+    # the sum's bound, then one rounding to 8 bits
+    assert ((D.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 4 * K ** 0.5 * 2.0 ** -24 * a.norm(dim=1)[:, None] * w.norm(dim=1)[None, :]).all()
 
 
+@GPU
 def test_gemm_wq_rows_do_not_mix(gpu):
     """an infinite activation spoils its own row only, also beside rows and K steps that a tile pads"""
     M, N, K = 40, 96, 768
@@ -80,6 +129,7 @@ def test_gemm_wq_rows_do_not_mix(gpu):
 @pytest.mark.parametrize("fmt,N,K", [(synth.Q4_K, 130, 256), (synth.Q4_K, 70, 768), (synth.Q5_K, 128, 512), (synth.IQ4_XS, 33, 768), (synth.Q8_0_SOA, 257, 192),
                                      (synth.Q5_1_SOA, 2560, 640), (synth.Q5_1_SOA, 100, 96), (synth.Q8_0_SOA, 40, 64)])
 @pytest.mark.parametrize("gather", [True, False])
+@GPU
 def test_grouped_tiles(gpu, fmt, N, K, gather):
     """every number of row blocks (tiles of 1, 31, 32, 33, 64, 65, 97, 128 rows), partial column blocks, K of a
     partial chunk of steps (Q8_0 K = 64 and 192) and Q5_1 rows that steps of 64 do not divide, routed and shared tiles"""
@@ -103,6 +153,7 @@ def test_grouped_tiles(gpu, fmt, N, K, gather):
 
 
 @pytest.mark.parametrize("N,K", [(64, 256), (70, 768), (1, 512), (130, 2048)])
+@GPU
 def test_gate_up_tiles(gpu, N, K):
     """the fused gate/up call at every number of row blocks and partial blocks of 64 rows: bit for bit the two
     grouped GEMMs and silu * up it stands for"""
