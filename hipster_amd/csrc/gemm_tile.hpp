@@ -125,7 +125,9 @@ __device__ __forceinline__ void wq_load(__amdgpu_buffer_rsrc_t b, uint32_t w, ui
         r.q = bld16(b, w + h16, 32u * t);
     }
 }
-// t0: the chunk's first step, a multiple of CK.  (A partial chunk of d, m or qh reads on past its stream.)
+// t0: the chunk's first step, a multiple of CK.  A partial chunk of d or m (K not in whole blocks of 256) reads up to 12 bytes
+// past its row, for the matrix's last row past the matrix: the step is in the vector offset there, which the resource's
+// range check counts by definition, dword by dword (gfx950 counts the scalar offset too).
 template <int F>
 __device__ __forceinline__ void wh_load(__amdgpu_buffer_rsrc_t b, uint32_t w, uint32_t h16, int K, uint32_t t0, WHead<F>& r) {
     const uint32_t nb = (uint32_t)K >> 8, k8 = (uint32_t)K >> 3, n = t0 >> 2;
@@ -142,10 +144,10 @@ __device__ __forceinline__ void wh_load(__amdgpu_buffer_rsrc_t b, uint32_t w, ui
         r.y[1] = bld16(b, w + h16, nb * 128u + 64u * n + 32u);
         r.d = bld2(b, w, nb * 208u + 2u * n);
     } else if constexpr (F == QMM_Q8_0_SOA) {
-        r.x = bld16(b, w, (uint32_t)K + 4u * t0);
+        r.x = bld16(b, w + (uint32_t)K + 4u * t0, 0);
     } else if constexpr (F == QMM_Q5_1_SOA) {
-        r.x = bld16(b, w, 5u * k8 + 4u * t0);
-        r.m = bld16(b, w, 5u * k8 + (k8 >> 1) + 4u * t0);
+        r.x = bld16(b, w + 5u * k8 + 4u * t0, 0);
+        r.m = bld16(b, w + 5u * k8 + (k8 >> 1) + 4u * t0, 0);
         r.y[0] = bld16(b, w, 4u * k8 + 8u * t0);
         r.y[1] = bld16(b, w, 4u * k8 + 8u * t0 + 16u);
     }

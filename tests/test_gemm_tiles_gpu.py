@@ -97,6 +97,23 @@ def test_gemm_wq_short_k(gpu, fmt, K):
     assert err(D, ref) <= K ** 0.5 * 2.0 ** -24
 
 
+@pytest.mark.parametrize("fmt,K", [(synth.Q8_0_SOA, 128), (synth.Q8_0_SOA, 640), (synth.Q5_1_SOA, 128), (synth.Q5_1_SOA, 896)])
+@GPU
+def test_bytes_behind_the_matrix_do_not_matter(gpu, fmt, K):
+    """a last chunk of scales that is not full, of the last row: what lies behind the matrix (scales of NaN here) is not
+    read into any result, in a tile by waves of 32 rows and in one by producers"""
+    for M, N in ((300, 4097), (5, 37)):
+        W = synth.matrix(7210 + K, fmt, N, K)
+        buf = torch.full((W.size + 256,), 255, dtype=torch.uint8, device="cuda")
+        buf[:W.size] = dev(W).reshape(-1)
+        A = torch.from_numpy(synth.normal_f32(7211, (M, K))).cuda().bfloat16()
+        D, E = (torch.full((M, N), float("nan"), device="cuda") for _ in range(2))
+        qmm.gemm_wq(fmt, buf[:W.size], A, D, M, N, K)
+        buf[W.size:] = 0
+        qmm.gemm_wq(fmt, buf[:W.size], A, E, M, N, K)
+        assert torch.isfinite(D).all() and torch.equal(D, E)
+
+
 @GPU
 def test_gemm_bf16_odd_step_count_and_strides(gpu):
     """K = 192 (three steps) and operands that are views of wider matrices, garbage (NaN) around them"""
@@ -113,10 +130,10 @@ def test_gemm_bf16_odd_step_count_and_strides(gpu):
     assert ((D.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 4 * K ** 0.5 * 2.0 ** -24 * a.norm(dim=1)[:, None] * w.norm(dim=1)[None, :]).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(40, 96, 768), (300, 4200, 256)])
 @GPU
-def test_gemm_wq_rows_do_not_mix(gpu):
+def test_gemm_wq_rows_do_not_mix(gpu, M, N, K):
     """an infinite activation spoils its own row only, also beside rows and K steps that a tile pads"""
-    M, N, K = 40, 96, 768
     A, W, Wb, ref = operands(synth.Q4_K, M, N, K, 7300)
     A[7, 5] = float("inf")
     D = torch.zeros((M, N), device="cuda")
