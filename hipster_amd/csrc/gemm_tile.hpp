@@ -333,9 +333,11 @@ __device__ __forceinline__ void gt_dma(__amdgpu_buffer_rsrc_t r, uint4* lds, uin
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, v, s, 0, 0);
 }
 
+static __device__ const uint8_t gt_zeros[16] __attribute__((aligned(16))) = {};      // steps past the end for 64-bit row offsets
+
 // One tile of 32 NRB rows x 32 CW columns, CW waves.  s0..s3: the ring's stages, at least 32 NRB * 8 slots each and separate __shared__ arrays: the compiler then knows which stage a DMA writes and an LDS read
 // waits for that stage only.  abase / wbase: the operands' tile, abytes / wbytes its extent; arow(r), woff: byte offsets of
-// A's row r and of the lane's weight row (column 32 cw + fr) in it; put(i, e, v): register e of row block i, which is row 32i + 8(e/4) + 4h + e%4, column 32 cw + fr.
+// A's row r and of the lane's weight row (column 32 cw + fr) in it (64-bit offsets of A go past the resource); put(i, e, v): register e of row block i, which is row 32i + 8(e/4) + 4h + e%4, column 32 cw + fr.
 template <int F, int NRB, int CW, class ARow, class Put>
 __device__ __forceinline__ void gemm_tile_core(uint4* s0, uint4* s1, uint4* s2, uint4* s3, const uint8_t* abase, uint32_t abytes,
                                                const uint8_t* wbase, uint32_t wbytes, uint32_t woff, int K, const ARow& arow,
@@ -345,7 +347,8 @@ __device__ __forceinline__ void gemm_tile_core(uint4* s0, uint4* s1, uint4* s2, 
     const int cw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nk = K >> 6;
     const uint32_t h16 = 16u * (uint32_t)h;
     // DMA instruction q of the stage fills slots 64q + lane: rows 8q..8q+7, slot column lane % 8
-    uint32_t aoff[ND];
+    using Off = decltype(arow(0));       // uint64_t: rows beyond a buffer offset's span
+    Off aoff[ND];
 #pragma unroll
     for (int i = 0; i < ND; ++i) {
         const int q = min(cw + CW * i, NI - 1), r = 8 * q + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
@@ -363,7 +366,11 @@ __device__ __forceinline__ void gemm_tile_core(uint4* s0, uint4* s1, uint4* s2, 
         uint4* st = stage(sc);
 #pragma unroll
         for (int i = 0; i < ND; ++i)
-            if (i >= i0 && i < i1 && (NI % CW == 0 || cw + CW * i < NI)) gt_dma(r, st + 64 * (cw + CW * i), aoff[i], 128u * (uint32_t)t);
+            if (i >= i0 && i < i1 && (NI % CW == 0 || cw + CW * i < NI)) {
+                uint4* dst = st + 64 * (cw + CW * i);
+                if constexpr (sizeof(Off) == 4) gt_dma(r, dst, aoff[i], 128u * (uint32_t)t);
+                else dma16((t < nk ? abase + 128u * (uint32_t)t : gt_zeros) + (t < nk ? aoff[i] : 0), lds_addr(dst));
+            }
     };
     WQ<F> raw[4];
     WHead<F> head;                                     // loaded with the first step of its chunk

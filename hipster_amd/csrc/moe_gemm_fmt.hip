@@ -156,18 +156,27 @@ __global__ void __launch_bounds__(256) k_moe_gemm_fmt(FArgs a, int part) {
     }
 }
 
-// A tile with a row beyond the span of a 32-bit buffer offset (an A of more than 3.75 GiB): each thread sums whole
-// output elements, straight from memory
-constexpr uint32_t kASpan = 0xf0000000u;
-template <int F>
-__device__ float far_dot(const uint16_t* x, const uint8_t* wrow, int K) {
-    float acc = 0.f;
-    for (int sb = 0; sb < K / 32; ++sb) {
-        float w[32];
-        dq_sub32<F>(wrow, K, sb, w);
-        for (int k = 0; k < 32; ++k) acc = __builtin_fmaf(bf2f(x[32 * sb + k]), bf2f(f2bf_bits(w[k])), acc);
-    }
-    return acc;
+// A's rows are gathered through 32-bit buffer offsets, which span 3.75 GiB.  A tile with a row further out runs the same
+// core with 64-bit row addresses: the same bits, its DMA in the flat form that the compiler's counts leave out, so that it
+// waits for more loads than it has to.  (Passes over windows of 3.75 GiB instead kept the addresses of every shape in registers
+// across the loop: one workgroup per CU instead of two, all tiles up to 1.8 times slower.)
+constexpr uint32_t kASpan = 0xf0000000u, kAPast = kASpan + 0x08000000u;      // kAPast: an offset out of range with a row's bytes added
+__device__ __forceinline__ bool a_far(const int* rows, uint32_t lda) {
+    return __syncthreads_or(threadIdx.x < FBM && ((unsigned long long)(unsigned)rows[threadIdx.x] + 1) * lda > kASpan);
+}
+// go(row blocks, byte offset of A's row r)
+template <class Go>
+__device__ __forceinline__ void each_shape(const int* rows, int n, uint32_t lda, const Go& go) {
+    auto shapes = [&](const auto& arow) __attribute__((always_inline)) {
+        switch ((n + 31) >> 5) {
+            case 1: go(std::integral_constant<int, 1>(), arow); break;
+            case 2: go(std::integral_constant<int, 2>(), arow); break;
+            case 3: go(std::integral_constant<int, 3>(), arow); break;
+            default: go(std::integral_constant<int, 4>(), arow); break;
+        }
+    };
+    if (a_far(rows, lda)) shapes([&](int r) { return (uint64_t)(uint32_t)rows[r] * lda; });       // (rows past the last repeat it)
+    else shapes([&](int r) { return r < n ? (uint32_t)rows[r] * lda : kAPast; });                 // past the span: zeros
 }
 
 template <int F>
@@ -183,31 +192,15 @@ __device__ __forceinline__ void moe_tile_unit(const FArgs& a, int part) {
     const uint32_t lda = 2u * (uint32_t)a.K, ldw = (uint32_t)fmt_row_bytes_rt(F, a.K);
     const uint8_t* wb = (tl.expert < 0 ? a.wsh : a.w + (size_t)tl.expert * a.ebytes) + (size_t)n0 * ldw;
     const uint32_t wbytes = (uint32_t)min(FBN, a.N - n0) * ldw;
-    const bool far = threadIdx.x < FBM && ((unsigned long long)(unsigned)rows[threadIdx.x] + 1) * lda > kASpan;
-    if (__syncthreads_or(far)) {
-        const int nn = min(FBN, a.N - n0);
-        for (int i = threadIdx.x; i < tl.ncols * nn; i += blockDim.x) {
-            const int r = i / nn, c = i - r * nn;
-            a.D[(size_t)(tl.k0 + r) * a.N + n0 + c] = far_dot<F>(a.A + (size_t)rows[r] * a.K, wb + (size_t)c * ldw, a.K);
-        }
-        return;
-    }
-    auto go = [&](auto nrb_c) {
+    each_shape(rows, tl.ncols, lda, [&](auto nrb_c, const auto& arow) __attribute__((always_inline)) {
         constexpr int NRB = decltype(nrb_c)::value;
         gemm_tile_core<F, NRB, FBN / 32>(
-            s0, s1, s2, s3, (const uint8_t*)a.A, kASpan, wb, wbytes, (uint32_t)(n - n0) * ldw, a.K,
-            [&](int r) { return r < tl.ncols ? (uint32_t)rows[r] * lda : kASpan + 0x08000000u; },   // past the span: zeros
+            s0, s1, s2, s3, (const uint8_t*)a.A, kASpan, wb, wbytes, (uint32_t)(n - n0) * ldw, a.K, arow,
             [&](int i, int e, float v) {
                 const int r = 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
                 if (r < tl.ncols && n < a.N) a.D[(size_t)(tl.k0 + r) * a.N + n] = v;
             });
-    };
-    switch ((tl.ncols + 31) >> 5) {
-        case 1: go(std::integral_constant<int, 1>()); break;
-        case 2: go(std::integral_constant<int, 2>()); break;
-        case 3: go(std::integral_constant<int, 3>()); break;
-        default: go(std::integral_constant<int, 4>()); break;
-    }
+    });
 }
 template <int F>
 __global__ void __launch_bounds__(256) k_moe_gemm_tile(FArgs a, int part) {
@@ -244,24 +237,13 @@ __device__ __forceinline__ void moe_gate_up_unit(const GuArgs& g) {
     const uint8_t* wg = (tl.expert < 0 ? a.wsh : a.w) + eo;
     const uint8_t* wu = (tl.expert < 0 ? g.wush : g.wu) + eo;
     const int nn = min(kGuRows, a.N - n0);
-    const bool far = threadIdx.x < FBM && ((unsigned long long)(unsigned)rows[threadIdx.x] + 1) * lda > kASpan;
-    if (__syncthreads_or(far)) {
-        for (int i = threadIdx.x; i < tl.ncols * nn; i += blockDim.x) {
-            const int r = i / nn, c = i - r * nn;
-            const uint16_t* x = a.A + (size_t)rows[r] * a.K;
-            g.H[(size_t)(tl.k0 + r) * a.N + n0 + c] = (uint16_t)f2bf_bits(
-                silu_mul(far_dot<QMM_Q4_K>(x, wg + (size_t)c * ldw, a.K), far_dot<QMM_Q4_K>(x, wu + (size_t)c * ldw, a.K)));
-        }
-        return;
-    }
     // an up wave's rows are its base's rows 64 .. 127 (wave 2, 3 of the core's four column blocks)
     const uint8_t* wb = up ? wu - (size_t)kGuRows * ldw : wg;
     const uint32_t wbytes = (uint32_t)(nn + (up ? kGuRows : 0)) * ldw;
-    auto go = [&](auto nrb_c) {
+    each_shape(rows, tl.ncols, lda, [&](auto nrb_c, const auto& arow) __attribute__((always_inline)) {
         constexpr int NRB = decltype(nrb_c)::value;
         gemm_tile_core<QMM_Q4_K, NRB, 4>(
-            s0, s1, s2, s3, (const uint8_t*)a.A, kASpan, wb, wbytes, (uint32_t)(32 * wave + (lane & 31)) * ldw, a.K,
-            [&](int r) { return r < tl.ncols ? (uint32_t)rows[r] * lda : kASpan + 0x08000000u; },
+            s0, s1, s2, s3, (const uint8_t*)a.A, kASpan, wb, wbytes, (uint32_t)(32 * wave + (lane & 31)) * ldw, a.K, arow,
             [&](gt_f32x16 (&acc)[NRB]) {
                 float* xch = (float*)(wave & 1 ? s1 : s0);          // the ring is no longer needed: NRB x 16 x 64 floats
                 __syncthreads();
@@ -283,13 +265,7 @@ __device__ __forceinline__ void moe_gate_up_unit(const GuArgs& g) {
                         }
                 }
             });
-    };
-    switch ((tl.ncols + 31) >> 5) {
-        case 1: go(std::integral_constant<int, 1>()); break;
-        case 2: go(std::integral_constant<int, 2>()); break;
-        case 3: go(std::integral_constant<int, 3>()); break;
-        default: go(std::integral_constant<int, 4>()); break;
-    }
+    });
 }
 __global__ void __launch_bounds__(256) k_moe_gate_up_tile(GuArgs a) { moe_gate_up_unit(a); }
 

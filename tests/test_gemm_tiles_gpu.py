@@ -193,3 +193,45 @@ def test_gate_up_tiles(gpu, N, K):
     qmm.moe_silu_bf16(gu[0], gu[1], h2, rows * N)
     assert torch.isfinite(h.float()).all() and h.float().abs().max() > 0
     assert torch.equal(h.view(torch.int16), h2.view(torch.int16))
+
+
+@pytest.mark.parametrize("fmt,K", [(synth.Q4_K, 768), (synth.Q5_K, 512), (synth.Q5_1_SOA, 640)])
+@GPU
+def test_grouped_rows_beyond_a_buffer_offset(gpu, fmt, K):
+    """an A of more than 3.75 GiB, the span of the gather's offsets: tiles of near, of far and of both kinds of rows give the
+    bits that the same rows give in a small A, gathered (the fused gate/up call too) and in sorted order"""
+    N, rows_a = 130, 0xf0000000 // (2 * K) + 4000
+    near, far = torch.arange(0, 200), torch.arange(rows_a - 300, rows_a)
+    sizes = [128, 64, 97, 128, 5]
+    g = synth.rng(7800)
+    pick = [near[:128], far[:64], torch.cat([near, far])[torch.from_numpy(g.permutation(500)[:97])],
+            torch.cat([near, far])[torch.from_numpy(g.permutation(500)[:128])], far[-5:]]
+    rt = torch.cat(pick).int().cuda()
+    E, starts = len(sizes) - 1, np.concatenate([[0], np.cumsum(sizes)[:-1]])
+    tiles = dev(np.array([[e, starts[e], sizes[e]] for e in range(E)] + [[-1, starts[E], sizes[E]]], np.int32))
+    counts = dev(np.array([E, 1], np.int32))
+    W, S = dev(synth.experts(7801, fmt, E, N, K)), dev(synth.matrix(7802, fmt, N, K))
+    A = torch.empty((rows_a, K), dtype=torch.bfloat16, device="cuda")
+    for r in (near, far):
+        A[r.cuda()] = (torch.from_numpy(synth.normal_f32(7803 + int(r[0]) % 7, (len(r), K))).cuda() * 1e-3).bfloat16()
+    small = A[rt.long()].contiguous()
+    n, eb = len(rt), W[0].numel()
+    D, D2 = (torch.full((n, N), float("nan"), device="cuda") for _ in range(2))
+    qmm.moe_gemm_bf16(fmt, fmt, W, S, eb, tiles, counts, E + 1, rt, A, D, N, K)
+    qmm.moe_gemm_bf16(fmt, fmt, W, S, eb, tiles, counts, E + 1, None, small, D2, N, K)
+    assert torch.isfinite(D2).all() and torch.equal(D.view(torch.int32), D2.view(torch.int32))
+    if fmt == synth.Q4_K:
+        H, H2 = (torch.full((n, N), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        qmm.moe_gemm_gate_up_bf16(fmt, fmt, W, S, W, S, eb, tiles, counts, E + 1, rt, A, H, N, K)
+        qmm.moe_gemm_gate_up_bf16(fmt, fmt, W, S, W, S, eb, tiles, counts, E + 1, None, small, H2, N, K)
+        assert torch.isfinite(H2.float()).all() and torch.equal(H.view(torch.int16), H2.view(torch.int16))
+    # sorted order: consecutive rows of A, the last of them far
+    k0 = rows_a - 300
+    one = dev(np.array([[0, k0, 128], [1, k0 + 128, 100]], np.int32))
+    big = torch.full((rows_a, 2), float("nan"), device="cuda")
+    qmm.moe_gemm_bf16(fmt, fmt, W[:, :2].contiguous(), S[:2].contiguous(), 2 * W[0, 0].numel(), one, dev(np.array([2, 0], np.int32)), 2, None, A, big, 2, K)
+    near2 = dev(np.array([[0, 0, 128], [1, 128, 100]], np.int32))
+    few = torch.full((228, 2), float("nan"), device="cuda")
+    qmm.moe_gemm_bf16(fmt, fmt, W[:, :2].contiguous(), S[:2].contiguous(), 2 * W[0, 0].numel(), near2, dev(np.array([2, 0], np.int32)), 2, None,
+                      A[k0:k0 + 228].contiguous(), few, 2, K)
+    assert torch.isfinite(few).all() and torch.equal(big[k0:k0 + 228].view(torch.int32), few.view(torch.int32))
