@@ -217,22 +217,24 @@ __device__ __forceinline__ void wh_decode(const WHead<F>& r, int t0, int nk, int
 // The raw quants of a step as its slices read them: q the first sub-block's, x the second's.  IQ4_XS and Q5_1 pack
 // weights l and l + 16 of a sub-block in a byte and lane half h loaded sub-block h: an exchange between the halves gives
 // each its 16 weights of both sub-blocks (the first's high nibbles against the second's low ones), one per byte.
-template <int F>
-__device__ __forceinline__ WQ<F> wq_open(const WQ<F>& r) {
+// In two parts, the words of slices 0, 2 and those of slices 1, 3.
+template <int F, int PART>
+__device__ __forceinline__ void wq_open(const WQ<F>& r, WQ<F>& o) {
     if constexpr (F == QMM_IQ4_XS || F == QMM_Q5_1_SOA) {
-        WQ<F> o;
         auto swap = [](uint32_t v, uint32_t& a, uint32_t& b) {
             const auto s = __builtin_amdgcn_permlane32_swap(v & 0x0f0f0f0fu, (v >> 4) & 0x0f0f0f0fu, false, false);
             a = s[0];
             b = s[1];
         };
-        swap(r.q.x, o.q.x, o.x.x);
-        swap(r.q.y, o.q.y, o.x.y);
-        swap(r.q.z, o.q.z, o.x.z);
-        swap(r.q.w, o.q.w, o.x.w);
-        return o;
-    } else {
-        return r;
+        if constexpr (PART == 0) {
+            swap(r.q.x, o.q.x, o.x.x);
+            swap(r.q.y, o.q.y, o.x.y);
+        } else {
+            swap(r.q.z, o.q.z, o.x.z);
+            swap(r.q.w, o.q.w, o.x.w);
+        }
+    } else if constexpr (PART == 0) {
+        o = r;
     }
 }
 
@@ -244,11 +246,11 @@ __device__ __forceinline__ void u4_bf16(uint32_t v, float s24, float c, gt_bf16x
     o[i + 2] = (__bf16)mix_hi(e, s24, c);
     o[i + 3] = (__bf16)mix_hi(d, s24, c);
 }
-// four bytes b -> bf16(s * (b - bias)): b as the f16 number 1024 + b, exactly, minus 1024 + bias
+// four bytes b -> bf16(s * (b - bias)): b as the f16 number 1024 + b (one byte permute a pair), exactly, minus 1024 + bias
 __device__ __forceinline__ void s4_bf16(uint32_t v, float s, float bias, gt_bf16x8& o, int i) {
     const gt_h2 k = {(_Float16)(1024.f + bias), (_Float16)(1024.f + bias)};
-    const uint32_t e = __builtin_bit_cast(uint32_t, __builtin_bit_cast(gt_h2, (v & 0x00ff00ffu) | 0x64006400u) - k);
-    const uint32_t d = __builtin_bit_cast(uint32_t, __builtin_bit_cast(gt_h2, ((v >> 8) & 0x00ff00ffu) | 0x64006400u) - k);
+    const uint32_t e = __builtin_bit_cast(uint32_t, __builtin_bit_cast(gt_h2, __builtin_amdgcn_perm(0x64646464u, v, 0x04020400u)) - k);
+    const uint32_t d = __builtin_bit_cast(uint32_t, __builtin_bit_cast(gt_h2, __builtin_amdgcn_perm(0x64646464u, v, 0x04030401u)) - k);
     o[i] = (__bf16)mix_lo(e, s, 0.f);
     o[i + 1] = (__bf16)mix_lo(d, s, 0.f);
     o[i + 2] = (__bf16)mix_hi(e, s, 0.f);
@@ -274,8 +276,8 @@ __device__ __forceinline__ gt_bf16x8 w_slice(const WQ<F>& r, const WDec& c, int 
                 const uint32_t nib = (s < 2 ? q : q >> 4) & 0x0f0f0f0fu;
                 const uint32_t v = nib | (((word(c.hi[0], w) >> (2 * u + (s >> 1))) & 0x01010101u) << 4);
                 u4_bf16(v, a, s < 2 ? c.c[u] : c.c2[u], o, 4 * i);
-            } else if constexpr (F == QMM_IQ4_XS) {      // levels as unsigned bytes: signed level ^ 0x80 = level + 128
-                s4_bf16(iq4_levels4(q) ^ 0x80808080u, a, 128.f, o, 4 * i);
+            } else if constexpr (F == QMM_IQ4_XS) {
+                s4_bf16(iq4_levels4(q, 0x80808080u), a, 128.f, o, 4 * i);
             } else if constexpr (F == QMM_Q6_K_SOA) {
                 const uint32_t nib = (q >> (4 * (u & 1))) & 0x0f0f0f0fu;
                 const uint32_t v = nib | (((word(c.hi[u >> 1], w) >> (4 * (u & 1) + 2 * (s >> 1))) & 0x03030303u) << 4);
@@ -398,7 +400,7 @@ __device__ __forceinline__ void gemm_tile_core(uint4* s0, uint4* s1, uint4* s2, 
                 cur.x = raw[(U + 3) % 4].x;
             }
         } else {
-            cur = wq_open<F>(raw[U]);
+            wq_open<F, 0>(raw[U], cur);
         }
     };
     auto frags = [&](auto sc, int s, gt_bf16x8 (&af)[NRB]) {
@@ -446,6 +448,7 @@ __device__ __forceinline__ void gemm_tile_core(uint4* s0, uint4* s1, uint4* s2, 
             else frags(gt_ic<UN>(), 0, afn);
             gt_bf16x8 wn;
             if (s < 3) {
+                if (s == 0) wq_open<F, 1>(raw[U], cur);
                 wn = w_slice<F>(cur, dec, U, s + 1);
             } else {
                 if constexpr (UN == 0) wh_decode<F>(head, t + 1, nk, h, dec);
@@ -629,8 +632,8 @@ __device__ __forceinline__ gt_bf16x8 u_frag(const UQ<F>& r, const UHead& hd, uin
     } else if constexpr (F == QMM_IQ4_XS) {
         const uint32_t sl = hd.h.y >> (8 * j + 4 * b), sh = hd.h.x >> (16 + 4 * j + 2 * b), n = 4 * (c >> 1);
         const float sc = h2f(hd.h.x) * (float)((int)((sl & 15u) | ((sh & 3u) << 4)) - 32);
-        s4_bf16(iq4_levels4((r.q[b].x >> n) & 0x0f0f0f0fu) ^ 0x80808080u, sc, 128.f, o, 0);
-        s4_bf16(iq4_levels4((r.q[b].y >> n) & 0x0f0f0f0fu) ^ 0x80808080u, sc, 128.f, o, 4);
+        s4_bf16(iq4_levels4((r.q[b].x >> n) & 0x0f0f0f0fu, 0x80808080u), sc, 128.f, o, 0);
+        s4_bf16(iq4_levels4((r.q[b].y >> n) & 0x0f0f0f0fu, 0x80808080u), sc, 128.f, o, 4);
     } else if constexpr (F == QMM_Q6_K_SOA) {
         const float sc = h2f(hd.x.z >> (16 * ((t >> 2) & 1))) * (float)(int8_t)((u ? hd.x.y : hd.x.x) >> (16 * b + 8 * (c >> 1)));
         const int n = 4 * u, hb = 4 * u + 2 * b;

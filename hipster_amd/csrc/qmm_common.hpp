@@ -55,12 +55,12 @@ __device__ __forceinline__ uint32_t byte8(uint32_t lo, uint32_t hi, int i) {
 // 8-11, 12-15
 constexpr uint32_t kIq4L0 = 0xBFAD9881u, kIq4L1 = 0xF6EADDCFu, kIq4H0 = 0x26190D01u, kIq4H1 = 0x71594535u;
 // four nibbles (one per byte, 0..15) -> four signed levels: one byte permute per half of the table,
-// then a per-byte select on bit 3
-__device__ __forceinline__ uint32_t iq4_levels4(uint32_t nib) {
+// then one that takes byte i of the half that bit 3 names; flip 0x80808080: levels + 128, unsigned
+__device__ __forceinline__ uint32_t iq4_levels4(uint32_t nib, uint32_t flip = 0u) {
     const uint32_t sel = nib & 0x07070707u;
-    const uint32_t lo = __builtin_amdgcn_perm(kIq4L1, kIq4L0, sel), hi = __builtin_amdgcn_perm(kIq4H1, kIq4H0, sel);
-    const uint32_t m = ((nib >> 3) & 0x01010101u) * 0xffu;
-    return (hi & m) | (lo & ~m);
+    const uint32_t lo = __builtin_amdgcn_perm(kIq4L1 ^ flip, kIq4L0 ^ flip, sel);
+    const uint32_t hi = __builtin_amdgcn_perm(kIq4H1 ^ flip, kIq4H0 ^ flip, sel);
+    return __builtin_amdgcn_perm(hi, lo, ((nib >> 1) & 0x04040404u) | 0x03020100u);
 }
 // Q6_K: 6-bit values (0..63, one per byte) -> signed q-32 per byte without carries between bytes.
 __device__ __forceinline__ uint32_t q6_signed(uint32_t q) { return (q + 0x60606060u) ^ 0x80808080u; }
