@@ -270,17 +270,17 @@ __global__ void __launch_bounds__(256) k_gemm(const uint16_t* __restrict__ A, co
 struct TileShape { int bm, bn, fixed, more; };       // rows, columns; ns for the launch, first loads and stores, the same for each further workgroup
 constexpr TileShape kTiles[] = {{16, 16, 4000, 0},      {32, 16, 3200, 1400},   {64, 16, 3400, 2400},   {48, 32, 4500, 1500},   {64, 32, 4700, 1600},
                                 {64, 64, 2600, 900},    {128, 64, 4500, 1800},  {64, 128, 2500, 3800},  {96, 128, 6100, 1800},  {128, 128, 7900, 1800},
-                                {160, 128, 8100, 2100}, {128, 256, 8500, 4800}, {192, 256, 10900, 8000}, {256, 256, 13200, 9200}};
+                                {160, 128, 8100, 2100}, {192, 128, 10500, 4700}, {128, 256, 8500, 4800}, {192, 256, 10900, 8000}, {256, 256, 13200, 9200}};
 constexpr int kNumTiles = (int)(sizeof(kTiles) / sizeof(kTiles[0]));
 struct StepNs { uint16_t first, more; };
 constexpr StepNs kStep[7][kNumTiles] = {
-    {{77, 74}, {104, 104}, {137, 131}, {161, 207}, {178, 228}, {360, 357}, {429, 430}, {463, 318}, {496, 398}, {540, 484}, {630, 573}, {931, 944}, {1278, 1243}, {1644, 1628}},   // Q4_K
-    {{103, 99}, {126, 130}, {161, 177}, {207, 243}, {226, 284}, {452, 441}, {523, 508}, {525, 369}, {537, 489}, {662, 545}, {716, 637}, {1090, 1145}, {1405, 1389}, {1726, 1695}},   // Q5_K
-    {{99, 75}, {125, 128}, {163, 159}, {185, 210}, {204, 231}, {336, 330}, {421, 411}, {555, 445}, {627, 485}, {711, 587}, {756, 668}, {1143, 1210}, {1453, 1461}, {1768, 1772}},   // IQ4_XS
-    {{141, 40}, {148, 119}, {172, 175}, {164, 204}, {177, 216}, {361, 347}, {423, 413}, {628, 460}, {704, 505}, {752, 582}, {802, 657}, {1173, 1207}, {1468, 1498}, {1810, 1747}},   // Q6_K
-    {{87, 90}, {112, 141}, {147, 181}, {211, 207}, {232, 226}, {390, 372}, {464, 440}, {550, 474}, {607, 517}, {642, 594}, {684, 676}, {1096, 1131}, {1382, 1399}, {1672, 1674}},   // Q8_0
-    {{109, 87}, {130, 143}, {166, 175}, {191, 239}, {210, 255}, {395, 371}, {462, 453}, {608, 439}, {686, 525}, {776, 578}, {813, 671}, {1236, 1234}, {1472, 1515}, {1780, 1755}},   // Q5_1
-    {{74, 88}, {103, 113}, {166, 168}, {202, 185}, {224, 211}, {352, 339}, {442, 442}, {612, 591}, {666, 664}, {727, 736}, {815, 824}, {1336, 1223}, {1521, 1537}, {1732, 1727}},   // bf16
+    {{77, 74}, {104, 104}, {137, 131}, {161, 207}, {178, 228}, {360, 357}, {429, 430}, {463, 318}, {496, 398}, {540, 484}, {630, 573}, {695, 721}, {931, 944}, {1278, 1243}, {1644, 1628}},   // Q4_K
+    {{103, 99}, {126, 130}, {161, 177}, {207, 243}, {226, 284}, {452, 441}, {523, 508}, {525, 369}, {537, 489}, {662, 545}, {716, 637}, {771, 842}, {1090, 1145}, {1405, 1389}, {1726, 1695}},   // Q5_K
+    {{99, 75}, {125, 128}, {163, 159}, {185, 210}, {204, 231}, {336, 330}, {421, 411}, {555, 445}, {627, 485}, {711, 587}, {756, 668}, {843, 847}, {1143, 1210}, {1453, 1461}, {1768, 1772}},   // IQ4_XS
+    {{141, 40}, {148, 119}, {172, 175}, {164, 204}, {177, 216}, {361, 347}, {423, 413}, {628, 460}, {704, 505}, {752, 582}, {802, 657}, {888, 848}, {1173, 1207}, {1468, 1498}, {1810, 1747}},   // Q6_K
+    {{87, 90}, {112, 141}, {147, 181}, {211, 207}, {232, 226}, {390, 372}, {464, 440}, {550, 474}, {607, 517}, {642, 594}, {684, 676}, {788, 832}, {1096, 1131}, {1382, 1399}, {1672, 1674}},   // Q8_0
+    {{109, 87}, {130, 143}, {166, 175}, {191, 239}, {210, 255}, {395, 371}, {462, 453}, {608, 439}, {686, 525}, {776, 578}, {813, 671}, {876, 853}, {1236, 1234}, {1472, 1515}, {1780, 1755}},   // Q5_1
+    {{74, 88}, {103, 113}, {166, 168}, {202, 185}, {224, 211}, {352, 339}, {442, 442}, {612, 591}, {666, 664}, {727, 736}, {815, 824}, {918, 868}, {1336, 1223}, {1521, 1537}, {1732, 1727}},   // bf16
 };
 constexpr int step_row(int f) { return f == QMM_W_BF16 ? 6 : f; }
 static_assert(QMM_Q4_K == 0 && QMM_Q5_K == 1 && QMM_IQ4_XS == 2 && QMM_Q6_K_SOA == 3 && QMM_Q8_0_SOA == 4 && QMM_Q5_1_SOA == 5, "");
@@ -348,8 +348,9 @@ int launch_gemm(GemmArgs a, hipStream_t s) {
         case 8: return launch_tile<F, OUT_BF16, 3, 4>(a, s);
         case 9: return launch_tile<F, OUT_BF16, 4, 4>(a, s);
         case 10: return launch_tile<F, OUT_BF16, 5, 4>(a, s);
-        case 11: return launch_tile<F, OUT_BF16, 4, 8>(a, s);
-        case 12: return launch_tile<F, OUT_BF16, 6, 8>(a, s);
+        case 11: return launch_tile<F, OUT_BF16, 6, 4>(a, s);
+        case 12: return launch_tile<F, OUT_BF16, 4, 8>(a, s);
+        case 13: return launch_tile<F, OUT_BF16, 6, 8>(a, s);
         default: return launch_tile<F, OUT_BF16, 8, 8>(a, s);
     }
 }
