@@ -10,8 +10,7 @@
 //   qmm_f32_to_bf16, qmm_bf16_to_f32, qmm_bf16_to_f32_seg, qmm_bf16_to_f32_seg2   gemm.hip:77-95
 //
 // qmm_gemm_wq and qmm_gemm_bf16 run the kernels of gemm_tile.hpp with the weight source as a template
-// argument; pick_tile below chooses the tile by the shape.  qmm_gemm_bf16_ld keeps a kernel without buffer
-// resources (256 x 256 tiles, register-staged two-stage LDS ring) for row strides that no resource spans.
+// argument; pick_tile below chooses the tile by the shape.
 #include "fmt_dequant.hpp"
 #include "gemm_tile.hpp"
 #include "qmm_common.hpp"
@@ -23,9 +22,6 @@
 
 namespace qmm {
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // ------------------------------------------------------------------------------------------
 // Bit-exact dequantisation to bf16 (engine/src/quant.h:43-53,65-80 arithmetic, then RNE to bf16 as
@@ -130,136 +126,6 @@ __global__ void k_bf16_to_f32_seg2(const uint16_t* __restrict__ x, const uint16_
 }
 
 // ------------------------------------------------------------------------------------------
-// bf16 x bf16 MFMA GEMM for row strides beyond the tile kernel's buffer resources.  Macro tile GBM x GBN = 256 x 256, K step 64, 4 waves as 2 x 2, each wave a
-// 128 x 128 tile = 8 x 8 MFMA tiles of 16 x 16 (256 f32 accumulators per lane, held in AGPRs).
-// LDS holds two stages of {A 256 x 64, W 256 x 64} bf16 with rows padded to 72 elements (144 B):
-// the 16-byte fragment reads of 16 consecutive rows then fall on 16 distinct 4-bank groups.
-// Step s: issue the global loads of step s+1 into registers, run the 128 MFMAs of step s from
-// stage s&1, write step s+1's registers into the other stage, barrier.
-constexpr int GBM = 256, GBN = 256, GBK = 64, GLD = GBK + 8;
-constexpr int kStageElems = (GBM + GBN) * GLD;                 // bf16 elements per stage
-constexpr size_t kGemmLds = 2 * (size_t)kStageElems * 2;     // bytes (147,456)
-
-// A tile loader: bf16 [M][K] row-major; thread t owns 16-byte column t%8 of rows t/8 + 32p
-struct ALoad {
-    uint4 r[8];
-    __device__ __forceinline__ void load(const uint16_t* __restrict__ A, int M, int lda, int m0, int k0) {
-        const int t = threadIdx.x;
-#pragma unroll
-        for (int p = 0; p < 8; ++p) {
-            const int m = min(m0 + 32 * p + (t >> 3), M - 1);
-            r[p] = ld16(A + (size_t)m * lda + k0 + 8 * (t & 7));
-        }
-    }
-    __device__ __forceinline__ void store(__bf16* La) const {
-        const int t = threadIdx.x;
-#pragma unroll
-        for (int p = 0; p < 8; ++p) *(uint4*)&La[(32 * p + (t >> 3)) * GLD + 8 * (t & 7)] = r[p];
-    }
-};
-
-// W tile loader, bf16 [N][K]: thread t copies the 64 elements of row n0+t
-struct BLoadBf16 {
-    uint4 r[8];
-    __device__ __forceinline__ void load(const uint16_t* __restrict__ W, int N, int ldw, int n0, int k0) {
-        const int n = min(n0 + (int)threadIdx.x, N - 1);
-        const uint16_t* p = W + (size_t)n * ldw + k0;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) r[i] = ld16(p + 8 * i);
-    }
-    __device__ __forceinline__ void store(__bf16* Lb, int) const {
-        uint4* dst = (uint4*)&Lb[threadIdx.x * GLD];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) dst[i] = r[i];
-    }
-};
-
-// tile id -> (m tile, n tile), XCD-aware: workgroup id i runs on XCD i % 8; give XCD x the
-// contiguous tile range [x * ntiles/8, (x+1) * ntiles/8) with M tiles fastest, so the M tiles that
-// share a weight tile share one L2.  Falls back to the plain order when the count is not a multiple of 8.
-__device__ __forceinline__ void tile_of(int bid, int mt, int nt, int& tm, int& tn) {
-    const int ntiles = mt * nt;
-    int id = bid;
-    if ((ntiles & 7) == 0) id = (bid & 7) * (ntiles >> 3) + (bid >> 3);
-    tm = id % mt;
-    tn = id / mt;
-}
-
-// 128 MFMAs of one K step from one LDS stage
-__device__ __forceinline__ void mfma_step(const __bf16* La, const __bf16* Lb, int wm, int wn, int fr, int fk, f32x4 (&acc)[8][8]) {
-#pragma unroll
-    for (int ks = 0; ks < GBK / 32; ++ks) {
-        bf16x8 af[8], bf[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) af[i] = *(const bf16x8*)&La[(128 * wm + 16 * i + fr) * GLD + 32 * ks + fk];
-#pragma unroll
-        for (int jn = 0; jn < 8; ++jn) bf[jn] = *(const bf16x8*)&Lb[(128 * wn + 16 * jn + fr) * GLD + 32 * ks + fk];
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-#pragma unroll
-            for (int jn = 0; jn < 8; ++jn) acc[i][jn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf[jn], acc[i][jn], 0, 0, 0);
-    }
-}
-
-// Step s: the global loads of step s+1 go out first, then the MFMAs of step s from LDS stage s&1,
-// then step s+1's registers are written (A copied, W dequantised) into the other stage.
-template <class BL, class WT, bool OUT_BF16>
-__global__ void __launch_bounds__(256) k_gemm(const uint16_t* __restrict__ A, const WT* __restrict__ W, void* __restrict__ D,
-                                              int M, int N, int K, int lda, int ldw) {
-    extern __shared__ __align__(16) uint8_t smem_raw[];
-    __bf16* const lds = (__bf16*)smem_raw;
-    const int mt = (M + GBM - 1) / GBM, nt = (N + GBN - 1) / GBN;
-    int tm, tn;
-    tile_of(blockIdx.x, mt, nt, tm, tn);
-    const int m0 = tm * GBM, n0 = tn * GBN;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave & 1, wn = wave >> 1;
-    const int nk = K / GBK;
-    ALoad al;
-    BL bl;
-    al.load(A, M, lda, m0, 0);
-    bl.load(W, N, ldw, n0, 0);
-    al.store(lds);
-    bl.store(lds + GBM * GLD, 0);
-    lds_barrier();
-    f32x4 acc[8][8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int jn = 0; jn < 8; ++jn) acc[i][jn] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int fr = lane & 15, fk = 8 * (lane >> 4);
-    for (int s = 0; s < nk; ++s) {
-        const __bf16* La = lds + (size_t)(s & 1) * kStageElems;
-        const bool more = s + 1 < nk;
-        if (more) {
-            al.load(A, M, lda, m0, (s + 1) * GBK);
-            bl.load(W, N, ldw, n0, (s + 1) * GBK);
-        }
-        mfma_step(La, La + GBM * GLD, wm, wn, fr, fk, acc);
-        if (more) {
-            __bf16* Sa = lds + (size_t)((s + 1) & 1) * kStageElems;
-            al.store(Sa);
-            bl.store(Sa + GBM * GLD, (s + 1) * GBK);
-        }
-        lds_barrier();
-    }
-    // epilogue: acc[i][jn][r] = D[m0 + 128wm + 16i + 4*(lane/16) + r][n0 + 128wn + 16jn + lane%16]
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int m = m0 + 128 * wm + 16 * i + 4 * (lane >> 4) + r;
-            if (m >= M) continue;
-#pragma unroll
-            for (int jn = 0; jn < 8; ++jn) {
-                const int n = n0 + 128 * wn + 16 * jn + fr;
-                if (n >= N) continue;
-                if constexpr (OUT_BF16) ((uint16_t*)D)[(size_t)m * N + n] = (uint16_t)f2bf_bits(acc[i][jn][r]);
-                else ((float*)D)[(size_t)m * N + n] = acc[i][jn][r];
-            }
-        }
-    }
-}
-// ------------------------------------------------------------------------------------------
 // Tile choice of the dequantising GEMM (gemm_tile.hpp).  Every tile runs the same chain of matrix instructions over K, so the
 // choice changes no bit: it may look at everything.  The busiest of the CUs gets q = ceil(tiles / CUs) workgroups, and a
 // step of 64 takes it about kStep[format][tile].first ns for one of them and .more for each further one (measured on 256
@@ -326,7 +192,24 @@ int launch_few(const GemmArgs& a, hipStream_t s) {
 template <int F, bool OUT_BF16>
 int launch_gemm(GemmArgs a, hipStream_t s) {
     const int tile = pick_tile(F, a);
-    if (tile < 0) return QMM_ERR_SHAPE;
+    if (tile < 0) {
+        // rows so far apart that no tile's fit a buffer resource (strides above 138 million elements): as many rows and
+        // columns at a time as do, down to one of each
+        auto most = [](int n, size_t ld, size_t row) { return row > 0xffffffffu ? 0 : (int)std::min<size_t>(n, (0xffffffffu - row) / ld + 1); };
+        const int m = most(a.M, a.lda, (size_t)a.K * 2), n = most(a.N, a.ldw, a.rowbytes);
+        if (m == 0 || n == 0) return QMM_ERR_SHAPE;
+        for (int m0 = 0; m0 < a.M; m0 += m)
+            for (int n0 = 0; n0 < a.N; n0 += n) {
+                GemmArgs p = a;
+                p.A += (size_t)m0 * a.lda;
+                p.W += (size_t)n0 * a.ldw;
+                p.D = (uint8_t*)a.D + ((size_t)m0 * a.ldd + n0) * (OUT_BF16 ? 2 : 4);
+                p.M = std::min(m, a.M - m0);
+                p.N = std::min(n, a.N - n0);
+                if (int e = launch_gemm<F, OUT_BF16>(p, s)) return e;
+            }
+        return QMM_OK;
+    }
     // rows past M and N read at an offset that is out of the tile's range (and stays so with a row's bytes added), or at
     // row 0 where the range leaves no such offset
     const TileShape& t = kTiles[tile];
@@ -424,7 +307,7 @@ int qmm_gemm_wq(int fmt, const void* W, const uint16_t* A, float* D, int M, int 
     if (!W || !A || !D) return QMM_ERR_NULL;
     // K % 256 for the block formats (K % 512 for Q6_K_SOA: an even block count keeps its streams dword
     // aligned), K % 128 for the 32-weight SoA formats
-    const int kg = (fmt == QMM_Q8_0_SOA || fmt == QMM_Q5_1_SOA) ? 2 * GBK : fmt == QMM_Q6_K_SOA ? 512 : 256;
+    const int kg = (fmt == QMM_Q8_0_SOA || fmt == QMM_Q5_1_SOA) ? 128 : fmt == QMM_Q6_K_SOA ? 512 : 256;
     if (M <= 0 || N <= 0 || K <= 0 || K % kg != 0) return QMM_ERR_SHAPE;
     const size_t rb = fmt_row_bytes_rt(fmt, K);
     const GemmArgs a{(const uint8_t*)A, (const uint8_t*)W, D, (uint32_t)K * 2u, (uint32_t)rb, (uint32_t)rb, M, N, K, N, 0, 0};
@@ -441,19 +324,13 @@ int qmm_gemm_wq(int fmt, const void* W, const uint16_t* A, float* D, int M, int 
 
 int qmm_gemm_bf16_ld(const uint16_t* A, int lda, const uint16_t* W, int ldw, uint16_t* D, int M, int N, int K, void* stream) {
     if (!A || !W || !D) return QMM_ERR_NULL;
-    if (M <= 0 || N <= 0 || K <= 0 || K % GBK != 0 || lda < K || ldw < K) return QMM_ERR_SHAPE;
+    if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0 || lda < K || ldw < K) return QMM_ERR_SHAPE;
     // 16-byte row pieces: both operands' rows start 16-byte aligned
     if (((uintptr_t)A | (uintptr_t)W) % 16 != 0 || lda % 8 != 0 || ldw % 8 != 0) return QMM_ERR_ARG;
-    // the DMA of A addresses rows with 32-bit element offsets
+    // the limit of the call since its first kernel, which addressed A with 32-bit element offsets; nothing needs it now
     if ((uint64_t)(M - 1) * (uint64_t)lda + (uint64_t)K > 0xffffffffull) return QMM_ERR_SHAPE;
-    const GemmArgs a{(const uint8_t*)A, (const uint8_t*)W, D, (uint32_t)lda * 2u, (uint32_t)ldw * 2u, (uint32_t)K * 2u, M, N, K, N, 0, 0};
-    if (pick_tile(QMM_W_BF16, a) >= 0) return launch_gemm<QMM_W_BF16, true>(a, (hipStream_t)stream);
-    // rows so far apart that no tile's span fits a buffer resource
-    const int grid = ((M + GBM - 1) / GBM) * ((N + GBN - 1) / GBN);
-    hipLaunchKernelGGL((k_gemm<BLoadBf16, uint16_t, true>), dim3(grid), dim3(256), kGemmLds, (hipStream_t)stream, A, W, (void*)D, M, N,
-                       K, lda, ldw);
-    QMM_LAUNCH_CHECK();
-    return QMM_OK;
+    return launch_gemm<QMM_W_BF16, true>(GemmArgs{(const uint8_t*)A, (const uint8_t*)W, D, (uint32_t)lda * 2u, (uint32_t)ldw * 2u, (uint32_t)K * 2u,
+                                                  M, N, K, N, 0, 0}, (hipStream_t)stream);
 }
 
 int qmm_gemm_tile(int fmt, int M, int N, int K) {

@@ -130,6 +130,28 @@ def test_gemm_bf16_odd_step_count_and_strides(gpu):
     assert ((D.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 4 * K ** 0.5 * 2.0 ** -24 * a.norm(dim=1)[:, None] * w.norm(dim=1)[None, :]).all()
 
 
+@GPU
+def test_gemm_bf16_rows_too_far_apart_for_any_tile(gpu):
+    """row strides of 160 and 155 million elements, of A and of W: 16 rows of either exceed a buffer resource, so the call runs in
+    parts; the bits of the same rows side by side"""
+    M, N, K = 20, 27, 192
+    lda, ldw = 160_000_000, 155_000_000
+    a = torch.from_numpy(synth.normal_f32(7220, (M, K))).cuda().bfloat16()
+    w = torch.from_numpy(synth.normal_f32(7221, (N, K))).cuda().bfloat16()
+    want, D = (torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    qmm.gemm_bf16(a, w, want, M, N, K)
+    buf = torch.empty(max((M - 1) * lda, (N - 1) * ldw) + K, dtype=torch.bfloat16, device="cuda")
+    A = buf.as_strided((M, K), (lda, 1))
+    A.copy_(a)
+    qmm.gemm_bf16_ld(A, lda, w, K, D, M, N, K)
+    assert torch.equal(D.view(torch.int16), want.view(torch.int16))
+    D.fill_(float("nan"))
+    W = buf.as_strided((N, K), (ldw, 1))
+    W.copy_(w)
+    qmm.gemm_bf16_ld(a, K, W, ldw, D, M, N, K)
+    assert torch.isfinite(D.float()).all() and torch.equal(D.view(torch.int16), want.view(torch.int16))
+
+
 @pytest.mark.parametrize("M,N,K", [(40, 96, 768), (300, 4200, 256)])
 @GPU
 def test_gemm_wq_rows_do_not_mix(gpu, M, N, K):
