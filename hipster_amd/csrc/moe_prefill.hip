@@ -1,6 +1,6 @@
 // moe_prefill.hip -- MoE prefill on gfx950: device-side expert sort (histogram, prefix scan, stable
-// scatter, tiles), the grouped expert GEMM over the sorted rows (Q4_K experts dequantised to bf16 in
-// LDS, bf16 MFMA), and silu(g)*u -> bf16.
+// scatter, tiles), the grouped expert GEMM over the sorted rows for Q4_K rows of one or two blocks (other
+// rows and formats: moe_gemm_fmt.hip), and silu(g)*u -> bf16.
 //
 // Entry points (C ABI, include/hipster_qmm.h) and what they replace in the reference:
 //   qmm_moe_sort        the host path of engine/src/qwen4exp.cpp:628-645 (blocking device->host
@@ -284,53 +284,10 @@ __global__ void __launch_bounds__(256) k_moe_rowtok(const int* __restrict__ kpos
 }
 
 // ------------------------------------------------------------------------------------------
-// Grouped expert GEMM.  Work unit = (tile, block of the expert's weight rows).  A tile holds up to
-// 128 sorted rows: D[k0 + r][n] = sum_k A[row(r)][k] * W_e[n][k] for r < ncols, row(r) =
-// rowtab[k0 + r] (or k0 + r), W_e the expert's Q4_K matrix (the shared matrix when expert < 0).
-//
-// 512 threads = 8 waves, two per SIMD, side by side along the weight rows: wave w owns one 32-wide
-// MFMA column block (256 weight rows per workgroup) and all NRB = ceil(ncols / 32) row blocks of
-// the tile, so every weight is dequantised once per workgroup, by the wave that multiplies it,
-// straight into MFMA operand registers; the two waves of a SIMD hide each other's waits.
-// v_mfma_f32_32x32x16_bf16 takes from lane l weight row l%32 and k = 8(l/32)..+7 of a 16-wide K
-// slice; which k those are is free as long as A agrees, and for a 64-wide K step (one qs pair j of a
-// block) they are the low nibbles of qs bytes 16h..16h+7 (slice 0) and 16h+8..16h+15 (slice 1) and the high
-// nibbles of the same bytes (slices 2, 3), h = l/32, as in gemm_tile.hpp.  A (gathered bf16 rows, DMA issued by waves 0-3) streams global -> LDS with
-// global_load_lds_dwordx4 through a ring of XST = 5 stages issued four steps ahead; the weight rows'
-// Q4_K blocks (144 contiguous bytes per row, so one DMA instruction covers about 7 rows: coalesced)
-// stream through a ring of block stages, DMA issued by waves 4-7: two stages (one block of 4 K steps
-// ahead) for tiles of 65-128 rows, three (two blocks ahead) for tiles of at most 64 rows, whose
-// smaller A stages leave the room.  A tile of few rows spends little time per step, so one block in
-// flight per CU would bound its weight stream at about 37 KB per memory latency.
-// The raw bytes of step t+1 are dequantised while the MFMAs of step t run.  A stage: 32 NRB rows x 8
-// chunks of 16 B, chunk c of row r in slot r*8 + (c ^ ((r >> 1) & 7)) (conflict-free fragment
-// reads); block stage: 256 rows x 144 B, row-major.  The A ring comes first in LDS, then the weight
-// ring.
-// Rows of one Q4_K block (K = 256) run here; gate and up, and longer rows, on the tile core of gemm_tile.hpp or on
-// k_moe_gemm_as below (qmm_moe_gemm_bf16 says which and why).
-constexpr int kXMaxK = 256;
-constexpr int XBM = 128, XBW = 256, XBK = 64, XST = 5, XTHREADS = 512;
-constexpr int kXA = XBM * XBK / 8;                          // 16-byte chunks per A stage (1024)
-constexpr int kXW = 9 * XBW;                                // chunks per weight block stage (2304)
-constexpr size_t kXLds = ((size_t)XST * kXA + 2 * (size_t)kXW) * 16;   // 155,648 B
-// ring geometry for tiles of NRB row blocks: chunks per A stage, weight block stages
-template <int NRB>
-struct XRing {
-    static constexpr int kA = 256 * NRB;
-    static constexpr int WST = NRB <= 2 ? 3 : 2;
-    static_assert(((size_t)XST * kA + (size_t)WST * kXW) * 16 <= kXLds, "ring exceeds the launch's LDS");
-};
-
-// s_waitcnt immediate for "vmcnt <= v" (expcnt, lgkmcnt unconstrained)
-constexpr int vmcnt_imm(int v) { return (v & 15) | (7 << 4) | (15 << 8) | ((v >> 4) << 14); }
-
-// wait until at most `rem` steps of L loads each are outstanding (rem = 0, 1 or 2)
-template <int L>
-__device__ __forceinline__ void wait_steps(int rem) {
-    if (rem >= 2) __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * L));
-    else if (rem == 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(L));
-    else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-}
+// Grouped expert GEMM for rows of one or two Q4_K blocks.  A tile holds up to 128 sorted rows:
+// D[k0 + r][n] = sum_k A[row(r)][k] * W_e[n][k] for r < ncols, row(r) = rowtab[k0 + r] (or k0 + r), W_e the
+// expert's Q4_K matrix (the shared matrix when expert < 0).
+constexpr int XBM = 128, XBW = 256;                         // rows of a tile, weight rows of a block
 
 struct XArgs {
     const uint8_t* w0;     // expert matrices, expert e at w0 + e * ebytes
@@ -341,10 +298,10 @@ struct XArgs {
     const int* rowtab;
     const uint16_t* A;
     void* D;               // f32 [k][ldd]
-    int N, K, nb;          // nb = weight-row blocks per tile
+    int N, nb;             // nb = 256-row weight blocks per tile
     int ldd;               // row stride of D (elements)
     int cap;               // capacity of tiles (the device count is clamped to it)
-    int bpu;               // k_moe_gemm_as: 256-row weight blocks per work unit
+    int bpu;               // weight blocks per work unit
 };
 
 // scales of K step j (qs pair j: sub-blocks 2j, 2j+1) of a Q4_K block header, pre-scaled for
@@ -361,230 +318,8 @@ __device__ __forceinline__ StepScl q4k_step_scales(const uint4 hd, int j) {
     return c;
 }
 
-template <int NRB>
-__device__ __forceinline__ void moe_gemm_tile(const XArgs& a, const qmm_moe_tile tl, int n0, uint4* As, const int* rows) {
-    constexpr int kA = XRing<NRB>::kA, WST = XRing<NRB>::WST;
-    uint4* const Ws = As + XST * kA;
-    const int lane = threadIdx.x & 63, fr = lane & 31, h = lane >> 5, fx = (fr >> 1) & 7;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), team = wave >> 2, wq = wave & 3;
-    const int K = a.K, N = a.N, nk = K / XBK, nblk = K >> 8;
-    const uint32_t rowbytes = (uint32_t)(K >> 8) * 144u;
-    const uint8_t* w0 = tl.expert >= 0 ? a.w0 + (size_t)tl.expert * a.ebytes : a.w0sh;
-    const uint32_t lA = lds_addr(As), lW = lds_addr(Ws);
-    // A DMA (waves 0-3): instruction q of wave wq fills slots (wq + 4q) * 64 + lane = row block q
-    uint32_t aoff[NRB];
-#pragma unroll
-    for (int q = 0; q < NRB; ++q) {
-        const int r = 8 * (wq + 4 * q) + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
-        aoff[q] = ((uint32_t)rows[r] * (uint32_t)K + (uint32_t)(8 * c)) * 2u;
-    }
-    // weight DMA (waves 4-7), one Q4_K block (144 B) of each of the 256 weight rows per 4 K steps:
-    // instruction k = 9 wq + q (0..35) fills chunks 64k + lane = row (64k + lane) / 9, 16-byte part
-    // (64k + lane) % 9.  
-    uint32_t woff[9];
-#pragma unroll
-    for (int q = 0; q < 9; ++q) {
-        const int k = 9 * wq + q, p = 64 * k + lane, row = p / 9, part = p - 9 * row;
-        woff[q] = (uint32_t)min(n0 + row, N - 1) * rowbytes + (uint32_t)(16 * part);
-    }
-    auto issue = [&](int p, int st) {       // A of step p (waves 0-3)
-        if (team == 0) {
-            const uint8_t* abase = (const uint8_t*)a.A + (size_t)p * (XBK * 2);
-            const uint32_t la = lA + (uint32_t)(st * kA * 16);
-#pragma unroll
-            for (int q = 0; q < NRB; ++q) dma16s(abase, aoff[q], la + (uint32_t)((wq + 4 * q) * 1024));
-        }
-    };
-    auto issue_w = [&](int b) {             // weight block b into block stage b % WST (waves 4-7)
-        if (team == 1) {
-            const uint32_t lw = lW + (uint32_t)((b % WST) * kXW * 16);
-#pragma unroll
-            for (int q = 0; q < 9; ++q) {
-                const int k = 9 * wq + q;
-                dma16s(w0 + b * 144, woff[q], lw + (uint32_t)(k * 1024));
-            }
-        }
-    };
-    // the lane's weight row (column slot of the stage) for its MFMA column block
-    const int c0 = 32 * wave + fr;
-    f32x16 acc[NRB];
-#pragma unroll
-    for (int i = 0; i < NRB; ++i)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc[i][e] = 0.f;
-    // A fragments of K slice s (16 wide) of the stage at la, row blocks 0..NRB-1
-    auto afrag = [&](const uint4* la, int s, bf16x8 (&af)[NRB]) {
-#pragma unroll
-        for (int i = 0; i < NRB; ++i) {
-            const uint4 v = la[(32 * i + fr) * 8 + ((4 * (s >> 1) + 2 * h + (s & 1)) ^ fx)];
-            af[i] = *(const bf16x8*)&v;
-        }
-    };
-    // raw weight bytes of one step for the lane's weight row, and their decode
-    struct Raw { uint4 hd, q; };
-    auto rawread = [&](int p, Raw& r) {     // step p: block p / 4, qs pair p % 4
-        const uint8_t* rp = (const uint8_t*)(Ws + ((p >> 2) % WST) * kXW) + c0 * 144;
-        const int j = p & 3;
-        r.hd = *(const uint4*)rp;
-        r.q = *(const uint4*)(rp + 16 + 32 * j + 16 * h);
-    };
-    // K slice s (16 wide) of the step: s 0, 1 = low nibbles of the two qs halves (sub-block 2j),
-    // s 2, 3 = their high nibbles (sub-block 2j+1)
-    auto deq = [&](const Raw& r, const StepScl& c, int s) {
-        const uint2 q = (s & 1) ? make_uint2(r.q.z, r.q.w) : make_uint2(r.q.x, r.q.y);
-        return s < 2 ? q4_bf16x8_mix(q.x, q.y, 0x000f000fu, c.sa, -c.ma) : q4_bf16x8_mix(q.x, q.y, 0x00f000f0u, c.sb, -c.mb);
-    };
-    // before dequantising step p (waves 4-7 hold at most WST - 1 blocks in flight: block b + WST - 1
-    // is issued at the first step of block b, after this wait, into the stage block b - 1 used)
-    auto wait_rem = [&](int rem, int p) {
-        if (team == 0) wait_steps<NRB>(rem);
-        else if ((p & 3) == 0) {
-            if (WST == 3 && (p >> 2) + 1 < nblk) __builtin_amdgcn_s_waitcnt(vmcnt_imm(9));
-            else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-        }
-    };
-    // prologue (K % 256 == 0, so nk >= 4): A steps 0..3 and weight blocks 0 (and 1) in flight, wait
-    // for A steps 0, 1 and block 0
-    issue(0, 0);
-    issue(1, 1);
-    issue(2, 2);
-    issue(3, 3);
-    issue_w(0);
-    if (WST == 3 && nblk > 1) issue_w(1);
-    wait_rem(2, 0);
-    lds_barrier();
-    bf16x8 wa[4], wb[4], af0[NRB];
-    {
-        Raw r;
-        rawread(0, r);
-        const StepScl c = q4k_step_scales(r.hd, 0);
-#pragma unroll
-        for (int s = 0; s < 4; ++s) wa[s] = deq(r, c, s);
-        afrag(As, 0, af0);
-    }
-    // Step t (t < nk-1): wait for step t+1's loads and barrier (t > 0); issue step t+4 into the
-    // stage step t-1 used; then 4 chunks (K slice s), each the NRB MFMAs of step t for slice s and
-    // the dequantisation of slice s of step t+1, fenced so that the MFMAs have VALU work of the same
-    // wave to overlap with.  A fragments are read one slice ahead, slice 0 of step t+1 during step t.
-    auto step = [&](int t, int st, int st1, int st4, const bf16x8 (&cur)[4], bf16x8 (&nxt)[4]) {
-        if (t > 0) {
-            wait_rem(min(nk - 1, t + 3) - (t + 1), t + 1);
-            lds_barrier();
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        const uint4* la = As + st * kA;
-        Raw r;
-        rawread(t + 1, r);
-        StepScl c;
-        bf16x8 af[NRB], afn[NRB];
-#pragma unroll
-        for (int i = 0; i < NRB; ++i) af[i] = af0[i];
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            if (s == 1) {       // DMA for step t+4 (its stage was last read in step t-1) after chunk 0's MFMAs
-                if (t + 4 < nk) issue(t + 4, st4);
-                if ((t & 3) == 0 && (t >> 2) + WST - 1 < nblk) issue_w((t >> 2) + WST - 1);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            afrag(s < 3 ? la : As + st1 * kA, s < 3 ? s + 1 : 0, afn);
-            if (s == 0) c = q4k_step_scales(r.hd, (t + 1) & 3);
-            nxt[s] = deq(r, c, s);
-            asm volatile("" : : "v"(nxt[s]));   // keeps the dequantisation inside this chunk
-#pragma unroll
-            for (int i = 0; i < NRB; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i], cur[s], acc[i], 0, 0, 0);
-            if (s == 0) {
-#pragma unroll
-                for (int k = 0; k < NRB; ++k) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, 44 / NRB + 1, 0);
-                }
-            } else {
-#pragma unroll
-                for (int k = 0; k < NRB; ++k) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, 24 / NRB + 1, 0);
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int i = 0; i < NRB; ++i) af[i] = afn[i];
-        }
-#pragma unroll
-        for (int i = 0; i < NRB; ++i) af0[i] = af[i];
-    };
-    int st = 0;
-    for (int t = 0; t < nk - 2; t += 2) {     // nk is a multiple of 4
-        const int s1 = st == XST - 1 ? 0 : st + 1, s2 = s1 == XST - 1 ? 0 : s1 + 1;
-        const int s3 = s2 == XST - 1 ? 0 : s2 + 1, s4 = s3 == XST - 1 ? 0 : s3 + 1, s5 = s4 == XST - 1 ? 0 : s4 + 1;
-        step(t, st, s1, s4, wa, wb);
-        step(t + 1, s1, s2, s5, wb, wa);
-        st = s2;
-    }
-    {   // steps nk-2 and nk-1
-        const int s1 = st == XST - 1 ? 0 : st + 1;
-        step(nk - 2, st, s1, 0, wa, wb);
-        const uint4* la = As + s1 * kA;
-        bf16x8 af[NRB];
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            if (s == 0) {
-#pragma unroll
-                for (int i = 0; i < NRB; ++i) af[i] = af0[i];
-            } else {
-                afrag(la, s, af);
-            }
-#pragma unroll
-            for (int i = 0; i < NRB; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i], wb[s], acc[i], 0, 0, 0);
-        }
-    }
-    // acc[i][e] = output row 32i + 8(e/4) + 4h + e%4 of the tile, weight row n0 + (column block) + fr
-    float* D = (float*)a.D;
-    const int n = n0 + 32 * wave + fr;
-#pragma unroll
-    for (int i = 0; i < NRB; ++i)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const int r = 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
-            if (r < tl.ncols && n < N) D[(size_t)(tl.k0 + r) * a.ldd + n] = acc[i][e];
-        }
-}
-
-// One workgroup per (tile, weight-row block).  Workgroup id i runs on XCD i % 8; XCD x takes tiles
-// x, x+8, x+16, ... with all their row blocks, so the blocks of one tile share its A rows in one L2.
-__global__ void __launch_bounds__(XTHREADS) k_moe_gemm_x(XArgs a) {
-    extern __shared__ __align__(16) uint8_t smem_raw[];
-    __shared__ int rows[XBM];
-    const int id = blockIdx.x, sid = id >> 3;
-    const int tix = 8 * (sid / a.nb) + (id & 7), nbi = sid % a.nb;
-    if (tix >= min(a.counts[0] + a.counts[1], a.cap)) return;
-    qmm_moe_tile tl = a.tiles[tix];
-    tl.ncols = max(1, min(tl.ncols, XBM));
-    if (threadIdx.x < XBM) {
-        const int k = tl.k0 + min((int)threadIdx.x, tl.ncols - 1);
-        rows[threadIdx.x] = a.rowtab ? a.rowtab[k] : k;
-    }
-    __syncthreads();
-    uint4* const As = (uint4*)smem_raw;
-    const int n0 = nbi * XBW;
-    switch ((tl.ncols + 31) >> 5) {
-        case 1: moe_gemm_tile<1>(a, tl, n0, As, rows); break;
-        case 2: moe_gemm_tile<2>(a, tl, n0, As, rows); break;
-        case 3: moe_gemm_tile<3>(a, tl, n0, As, rows); break;
-        default: moe_gemm_tile<4>(a, tl, n0, As, rows); break;
-    }
-}
-
-int launch_moe_gemm_x(const XArgs& a, int max_tiles, hipStream_t s) {
-    const int grid = 8 * ((max_tiles + 7) / 8) * a.nb;
-    hipLaunchKernelGGL(k_moe_gemm_x, dim3(grid), dim3(XTHREADS), kXLds, s, a);
-    QMM_LAUNCH_CHECK();
-    return QMM_OK;
-}
-
-// ------------------------------------------------------------------------------------------
-// Grouped expert GEMM with the tile's activations resident in LDS, for K = 512 (the MoE down
-// projection).  Work unit = (tile, run of bpu consecutive 256-row weight blocks).  The tile's A rows
-// (at most 128 x 512 bf16 = 128 KiB) are copied global -> LDS once per unit; after that every wave
+// The tile's activations are resident in LDS: K = 256 KB, KB = 2 (the MoE down projection) or 1.  Work unit = (tile, run
+// of bpu consecutive 256-row weight blocks).  The tile's A rows (at most 128 x 512 bf16 = 128 KiB) are copied global -> LDS once per unit; after that every wave
 // works alone: it streams its own 32 weight rows of each block straight into registers, dequantises
 // them and multiplies them against A fragments read from LDS, block after block, and stores each
 // block's f32 results.  The main loop has no workgroup barrier and no LDS writes, and A is read from
@@ -594,12 +329,13 @@ int launch_moe_gemm_x(const XArgs& a, int max_tiles, hipStream_t s) {
 // two 8-byte pieces it cost the address units twice the instructions: 112 -> 106 us at 2048 tokens), slices 0
 // and 1 their low nibbles, slices 2 and 3 their high nibbles, and the A fragment of slice s is chunk
 // 4 (s / 2) + 2h + s % 2 of the step.  Two weight blocks per unit: 104.8 / 47.3 / 27.2 us at 2048 / 512 / 96 tokens
-// against 106.4 / 53.9 / 29.2 with four, whose units were too few for the CUs.  A in LDS: row r at r * 1040 bytes
-// (64 chunks of 16 B and 16 B of padding), so the 16 rows a quarter-wave reads fall in 16 distinct
+// against 106.4 / 53.9 / 29.2 with four, whose units were too few for the CUs.  A in LDS: row r at r * (512 KB + 16)
+// bytes, so the 16 rows a quarter-wave reads fall in 16 distinct
 // bank groups and every fragment address is one lane base plus a constant; one DMA instruction
 // copies one row.
-constexpr int kAsK = 512, kAsThreads = 512, kAsBlocksPerUnit = 2, kAsRowBytes = 1040;
-constexpr bool kAsDeferStores = false;
+constexpr int kAsThreads = 512;
+template <int KB>
+constexpr int kAsRowBytes = 512 * KB + 16;
 
 // f32 store the compiler does not see (address = wave-uniform base in SGPRs + per-lane 32-bit byte
 // offset): its waits for the weight loads issued before it are then computed over loads only (loads
@@ -615,25 +351,26 @@ __device__ __forceinline__ void st_f32_nc(const uint8_t* base, uint32_t voff, fl
 // 16h.. of pair j)
 struct AsRaw { uint4 hd, q0, q1, q2, q3; };
 
-template <int NRB>
+template <int NRB, int KB>
 __device__ __forceinline__ void moe_as_unit(const XArgs& a, const qmm_moe_tile tl, int b0, int b1, const int* rows,
                                             uint8_t* As) {
     const int lane = threadIdx.x & 63, fr = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    constexpr uint32_t rowbytes = 2 * 144u;          // two Q4_K blocks per weight row
+    constexpr uint32_t rowbytes = KB * 144u;
+    constexpr int kRow = kAsRowBytes<KB>;
     const int N = a.N;
     const uint8_t* w = tl.expert >= 0 ? a.w0 + (size_t)tl.expert * a.ebytes : a.w0sh;
-    {   // A rows 0 .. 32 NRB - 1 -> LDS, one DMA instruction (64 lanes x 16 B) per row
+    if (lane < 32 * KB) {   // A rows 0 .. 32 NRB - 1 -> LDS, one DMA instruction (16 B a lane) per row
         const uint32_t la = lds_addr(As);
         for (int r = wave; r < NRB * 32; r += 8)
-            dma16((const uint8_t*)a.A + ((size_t)rows[r] * kAsK + (size_t)(8 * lane)) * 2, la + (uint32_t)(r * kAsRowBytes));
+            dma16((const uint8_t*)a.A + ((size_t)rows[r] * (256 * KB) + (size_t)(8 * lane)) * 2, la + (uint32_t)(r * kRow));
     }
-    // group g = Q4_K block g % 2 of weight block b0 + g / 2; the lane's row in it (clamped: rows past
+    // group g = Q4_K block g % KB of weight block b0 + g / KB; the lane's row in it (clamped: rows past
     // N load row N-1 and are not stored)
-    const int nblk = b1 - b0, ng = 2 * nblk;
+    const int ng = KB * (b1 - b0);
     auto load = [&](int g, AsRaw& r) {
-        const int b = b0 + (g >> 1);
-        const uint8_t* p = w + (size_t)min(b * 256 + 32 * wave + fr, N - 1) * rowbytes + (size_t)(g & 1) * 144;
+        const int b = b0 + g / KB;
+        const uint8_t* p = w + (size_t)min(b * 256 + 32 * wave + fr, N - 1) * rowbytes + (size_t)(g % KB) * 144;
         const uint8_t* pq = p + 16 + 16 * h;
         r.hd = ld16(p);
         r.q0 = ld16(pq);
@@ -641,23 +378,23 @@ __device__ __forceinline__ void moe_as_unit(const XArgs& a, const qmm_moe_tile t
         r.q2 = ld16(pq + 64);
         r.q3 = ld16(pq + 96);
     };
-    f32x16 acc0[NRB], acc1[NRB];
+    f32x16 acc[NRB];
 #pragma unroll
     for (int i = 0; i < NRB; ++i)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc0[i][e] = acc1[i][e] = 0.f;
+        for (int e = 0; e < 16; ++e) acc[i][e] = 0.f;
     AsRaw ra, rb;
     load(0, ra);
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));      // the A copy has landed (and group 0)
+    __builtin_amdgcn_s_waitcnt(0);      // the A copy has landed (and group 0)
     __syncthreads();
     // lane bases: row fr (row blocks 0, 1) and row 64 + fr (row blocks 2, 3), chunk 2h
     typedef __attribute__((address_space(3))) const uint8_t lds_u8;
-    const lds_u8* alo = (const lds_u8*)As + fr * kAsRowBytes + 32 * h;
-    const lds_u8* ahi = alo + 64 * kAsRowBytes;
+    const lds_u8* alo = (const lds_u8*)As + fr * kRow + 32 * h;
+    const lds_u8* ahi = alo + 64 * kRow;
     asm volatile("" : "+v"(ahi));     // a base of its own: otherwise folded into alo + offsets past 64 KiB
 
-    // K step t (0..7) of the row; the four slices' NRB MFMAs each
-    auto step = [&](const uint4 q, const StepScl& c, int t, f32x16 (&acc)[NRB]) {
+    // K step t of the row; the four slices' NRB MFMAs each
+    auto step = [&](const uint4 q, const StepScl& c, int t) {
         bf16x8 wv[4];
         wv[0] = q4_bf16x8_mix(q.x, q.y, 0x000f000fu, c.sa, -c.ma);
         wv[1] = q4_bf16x8_mix(q.z, q.w, 0x000f000fu, c.sa, -c.ma);
@@ -670,7 +407,7 @@ __device__ __forceinline__ void moe_as_unit(const XArgs& a, const qmm_moe_tile t
             const int off = (8 * t + 4 * (s >> 1) + (s & 1)) * 16;
 #pragma unroll
             for (int i = 0; i < NRB; ++i)
-                v[i] = *(const __attribute__((address_space(3))) u32x4*)((i < 2 ? alo : ahi) + (i & 1) * 32 * kAsRowBytes + off);
+                v[i] = *(const __attribute__((address_space(3))) u32x4*)((i < 2 ? alo : ahi) + (i & 1) * 32 * kRow + off);
         };
         rd(af, 0);
 #pragma unroll
@@ -687,7 +424,7 @@ __device__ __forceinline__ void moe_as_unit(const XArgs& a, const qmm_moe_tile t
     // results of weight block b (tile row 32i + 8(e/4) + e%4 + 4h): the uniform row part walks a
     // scalar pointer (kept opaque, so its 64 values are formed one at a time instead of hoisted out of
     // the loop), the lane part (4h rows, column n) is a fixed byte offset; then the set restarts at 0
-    auto store = [&](f32x16 (&acc)[NRB], int b) {
+    auto store = [&](int b) {
         const int n = b * 256 + 32 * wave + fr;
         const uint32_t voff = (uint32_t)(4 * h * a.ldd + n) * 4u;
         int rem = n < N ? tl.ncols - 4 * h : 0;     // the lane stores uniform row offsets below rem
@@ -704,49 +441,33 @@ __device__ __forceinline__ void moe_as_unit(const XArgs& a, const qmm_moe_tile t
                 p += (e & 3) == 3 ? 5 * rs : rs;     // next row: +1, or +5 after the 4th of a group of 8
             }
     };
-    // group g (Q4_K block kb = g % 2 of its weight block): the K steps of raw r into acc; the next
-    // group's loads go out after the first step.  Deferred stores: the previous block's set accp is
-    // stored after the first step of a block's first group (the wait for the next weights, three
-    // steps later, then finds those stores drained); otherwise a block's set is stored at its end.
+    // group g (Q4_K block kb of its weight block): the K steps of raw r; the next group's loads go out after
+    // the first step, a weight block's results are stored behind its last group.
     // Fenced steps: hoisting a step's A fragments and dequantisation over the previous step's MFMAs
     // runs out of registers.
-    auto group = [&](int g, int kb, const AsRaw& r, AsRaw& fill, f32x16 (&acc)[NRB], f32x16 (&accp)[NRB]) {
+    auto group = [&](int g, int kb, const AsRaw& r, AsRaw& fill) {
         const int t0 = 4 * kb;
-        step(r.q0, q4k_step_scales(r.hd, 0), t0, acc);
+        step(r.q0, q4k_step_scales(r.hd, 0), t0);
         __builtin_amdgcn_sched_barrier(0);
         load(min(g + 1, ng - 1), fill);
-        if (kAsDeferStores && kb == 0 && g > 0) store(accp, b0 + (g >> 1) - 1);
         __builtin_amdgcn_sched_barrier(0);
-        step(r.q1, q4k_step_scales(r.hd, 1), t0 + 1, acc);
+        step(r.q1, q4k_step_scales(r.hd, 1), t0 + 1);
         __builtin_amdgcn_sched_barrier(0);
-        step(r.q2, q4k_step_scales(r.hd, 2), t0 + 2, acc);
+        step(r.q2, q4k_step_scales(r.hd, 2), t0 + 2);
         __builtin_amdgcn_sched_barrier(0);
-        step(r.q3, q4k_step_scales(r.hd, 3), t0 + 3, acc);
+        step(r.q3, q4k_step_scales(r.hd, 3), t0 + 3);
         __builtin_amdgcn_sched_barrier(0);
-        if (!kAsDeferStores && kb == 1) store(acc, b0 + (g >> 1));
+        if (kb == KB - 1) store(b0 + g / KB);
     };
-    if constexpr (kAsDeferStores) {
-        // blocks in pairs: acc0 for even blocks, acc1 for odd ones
-        for (int bi = 0; bi < nblk; bi += 2) {
-            group(2 * bi, 0, ra, rb, acc0, acc1);
-            group(2 * bi + 1, 1, rb, ra, acc0, acc1);
-            if (bi + 1 < nblk) {
-                group(2 * bi + 2, 0, ra, rb, acc1, acc0);
-                group(2 * bi + 3, 1, rb, ra, acc1, acc0);
-            }
-        }
-        if ((nblk - 1) & 1) store(acc1, b1 - 1);
-        else store(acc0, b1 - 1);
-    } else {
-        for (int bi = 0; bi < nblk; ++bi) {
-            group(2 * bi, 0, ra, rb, acc0, acc1);
-            group(2 * bi + 1, 1, rb, ra, acc0, acc1);
-        }
+    for (int g = 0; g < ng; g += 2) {
+        group(g, 0, ra, rb);
+        if (KB == 2 || g + 1 < ng) group(g + 1, KB - 1, rb, ra);
     }
 }
 
 // One workgroup per (tile, run of bpu weight blocks); workgroup id i runs on XCD i % 8 and XCD x
 // takes tiles x, x+8, ... with all their runs (the runs of a tile share its A rows in one L2).
+template <int KB>
 __global__ void __launch_bounds__(kAsThreads) k_moe_gemm_as(XArgs a) {
     extern __shared__ __align__(16) uint8_t smem_raw[];
     __shared__ int rows[XBM];
@@ -763,17 +484,18 @@ __global__ void __launch_bounds__(kAsThreads) k_moe_gemm_as(XArgs a) {
     __syncthreads();
     const int b0 = ui * a.bpu, b1 = min(a.nb, b0 + a.bpu);
     switch ((tl.ncols + 31) >> 5) {
-        case 1: moe_as_unit<1>(a, tl, b0, b1, rows, smem_raw); break;
-        case 2: moe_as_unit<2>(a, tl, b0, b1, rows, smem_raw); break;
-        case 3: moe_as_unit<3>(a, tl, b0, b1, rows, smem_raw); break;
-        default: moe_as_unit<4>(a, tl, b0, b1, rows, smem_raw); break;
+        case 1: moe_as_unit<1, KB>(a, tl, b0, b1, rows, smem_raw); break;
+        case 2: moe_as_unit<2, KB>(a, tl, b0, b1, rows, smem_raw); break;
+        case 3: moe_as_unit<3, KB>(a, tl, b0, b1, rows, smem_raw); break;
+        default: moe_as_unit<4, KB>(a, tl, b0, b1, rows, smem_raw); break;
     }
 }
 
-int launch_moe_gemm_as(XArgs a, int max_tiles, hipStream_t s) {
+template <int KB>
+int launch_moe_gemm_as(const XArgs& a, int max_tiles, hipStream_t s) {
     const int nu = (a.nb + a.bpu - 1) / a.bpu;
     const int grid = 8 * ((max_tiles + 7) / 8) * nu;
-    hipLaunchKernelGGL(k_moe_gemm_as, dim3(grid), dim3(kAsThreads), (size_t)XBM * kAsRowBytes, s, a);
+    hipLaunchKernelGGL(k_moe_gemm_as<KB>, dim3(grid), dim3(kAsThreads), (size_t)XBM * kAsRowBytes<KB>, s, a);
     QMM_LAUNCH_CHECK();
     return QMM_OK;
 }
@@ -839,18 +561,17 @@ int qmm_moe_gemm_bf16(int fmt, int shared_fmt, const void* W, const void* Wsh, s
     if (!W || !Wsh || !tiles || !counts || !A || !D) return QMM_ERR_NULL;
     if (N <= 0 || K <= 0 || K % kgran(fmt) != 0 || K % kgran(shared_fmt) != 0 || max_tiles < 0) return QMM_ERR_SHAPE;
     if (max_tiles == 0) return QMM_OK;
-    // Q4_K (2048 rows, 256 experts, top 8; this kernel against the tile core, us at 96 / 2048 / 4096 tokens): K = 256
-    // k_moe_gemm_x 17.0 / 76 / 127 against 16.4 / 85 / 145 (four K steps: the work around them decides, and its
-    // workgroups are twice as wide), K = 512 k_moe_gemm_as 20 / 88 / 153 against 21 / 110 / 196; from K = 768 on the core
-    // (30 / 142 / 233 with k_moe_gemm_x against 25 / 143 / 243, at K = 1536 49 / 250 / 391 against 48 / 228 / 381).
-    // All three take k in the same order: the same bits.
-    if (fmt != QMM_Q4_K || shared_fmt != QMM_Q4_K || (K != kAsK && K != kXMaxK))
+    // Q4_K (2048 rows, 256 experts, top 8; k_moe_gemm_as against the tile core, us at 96 / 2048 / 4096 tokens): K = 256
+    // 11 / 50 / 95 against 16 / 85 / 145, K = 512 17 / 80 / 145 against 21 / 110 / 196: A is read once for two weight blocks and no
+    // wave waits for another.  Longer rows do not fit in LDS.  Both take k in the same order: the same bits.
+    if (fmt != QMM_Q4_K || shared_fmt != QMM_Q4_K || K > 512)
         return launch_moe_gemm_fmt(fmt, shared_fmt, W, Wsh, ebytes, tiles, counts, max_tiles, rowtab, A, D, N, K,
                                    (hipStream_t)stream);
-    XArgs a{(const uint8_t*)W, (const uint8_t*)Wsh, ebytes, tiles, counts, rowtab, A, D, N, K,
-            (N + XBW - 1) / XBW, N, max_tiles, kAsBlocksPerUnit};
-    if (K == kAsK) return launch_moe_gemm_as(a, max_tiles, (hipStream_t)stream);
-    return launch_moe_gemm_x(a, max_tiles, (hipStream_t)stream);
+    // two weight blocks a unit; one where rows of one block and at most four of those leave a tile too few units (1000 x 256,
+    // 64 experts, 96 / 512 / 4096 tokens 7.2 / 12.9 / 37.6 against 10.1 / 13.4 / 34.8; 2048 x 256 12.5 / 25.1 / 113 against 11.3 / 23.7 / 96)
+    const int nb = (N + XBW - 1) / XBW, bpu = K == 256 && nb <= 4 ? 1 : 2;
+    const XArgs a{(const uint8_t*)W, (const uint8_t*)Wsh, ebytes, tiles, counts, rowtab, A, D, N, nb, N, max_tiles, bpu};
+    return K == 512 ? launch_moe_gemm_as<2>(a, max_tiles, (hipStream_t)stream) : launch_moe_gemm_as<1>(a, max_tiles, (hipStream_t)stream);
 }
 
 int qmm_moe_gemm_gate_up_bf16(int fmt, int shared_fmt, const void* Wg, const void* Wgsh, const void* Wu, const void* Wush,

@@ -19,7 +19,7 @@ import pytest
 ROOT = os.path.abspath(os.path.join(os.path.dirname(__file__), ".."))
 CSRC = os.path.join(ROOT, "hipster_amd", "csrc")
 HIPCC = "/opt/rocm/bin/hipcc"
-FILES = ["moe_prefill.hip", "router.hip"]      # the sources with inline-assembly memory instructions
+FILES = ["moe_prefill.hip", "moe_gemm_fmt.hip", "router.hip"]      # the sources with inline-assembly memory instructions
 
 
 def device_asm(src, tmp_path):
@@ -74,11 +74,11 @@ def test_inline_asm_memory_blocks_start_with_nop(asm):
             blocks.append([x for x in cur if x and not x.startswith(";")])
         elif inasm:
             cur.append(l)
-    # the loads (DMA into LDS) carry the guard; the scalar-base stores of the K = 512 grouped GEMM do
+    # the loads (DMA into LDS) carry the guard; the scalar-base stores of the Q4_K grouped GEMM of one or two blocks do
     # not (their base is only ever advanced by scalar adds: the second test checks that)
     mem = [b for b in blocks if any(x.startswith(("global_load", "buffer_load")) for x in b)]
-    if name == "moe_prefill.hip":
-        assert len(mem) > 100
+    # (the test finds them: one loop per number of row blocks and of blocks a row; one per row block, stage and format)
+    assert len(mem) >= {"moe_prefill.hip": 8, "moe_gemm_fmt.hip": 100, "router.hip": 1}[name]
     bad = [b for b in mem if not b[0].startswith("s_nop 4")]
     assert not bad, bad[:3]
 

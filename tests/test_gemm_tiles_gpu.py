@@ -217,12 +217,12 @@ def test_gate_up_tiles(gpu, N, K):
     assert torch.equal(h.view(torch.int16), h2.view(torch.int16))
 
 
-@pytest.mark.parametrize("fmt,K", [(synth.Q4_K, 768), (synth.Q5_K, 512), (synth.Q5_1_SOA, 640)])
+@pytest.mark.parametrize("fmt,K", [(synth.Q4_K, 256), (synth.Q4_K, 512), (synth.Q4_K, 768), (synth.Q5_K, 512), (synth.Q5_1_SOA, 640)])
 @GPU
 def test_grouped_rows_beyond_a_buffer_offset(gpu, fmt, K):
-    """an A of more than 3.75 GiB, the span of the gather's offsets: tiles of near, of far and of both kinds of rows give the
+    """an A of more than 4 GiB, past the span of the gather's 32-bit offsets: tiles of near, of far and of both kinds of rows give the
     bits that the same rows give in a small A, gathered (the fused gate/up call too) and in sorted order"""
-    N, rows_a = 130, 0xf0000000 // (2 * K) + 4000
+    N, rows_a = 130, 2 ** 32 // (2 * K) + 4000
     near, far = torch.arange(0, 200), torch.arange(rows_a - 300, rows_a)
     sizes = [128, 64, 97, 128, 5]
     g = synth.rng(7800)
