@@ -14,6 +14,7 @@
 // hot calls go to the tuned kernels of gemv.hip / moe_prefill.hip; these keep the remaining call
 // sites working with the reference's exact (not bf16-rounded) numerics.
 #include "fmt_unit.hpp"
+#include "q4k_pair.hpp"
 #include "qmm_common.hpp"
 
 #include <hip/hip_runtime.h>
@@ -228,9 +229,9 @@ __device__ __forceinline__ void qm_x_store(QmLds& L, int buf, const QmXRegs<CB>&
     }
 }
 
-// a lane's quants of a block: 16-byte piece kq of each couple of qs pairs (64 bytes).  As four 8-byte pieces, one a
-// pair, they were five loads a row and block instead of three, each touching 16 rows, and the address units set the
-// time (512 tokens, 16-column tiles: gate, up and down 292 -> 263 us with the activation passes between them).
+// a lane's quants of a block: 16-byte piece kq of each couple of qs pairs (couple_split).  As four 8-byte pieces they were
+// five loads a row and block instead of three (512 tokens, 16-column tiles: gate, up and down 292 -> 263 us with the
+// activation passes between them).
 struct QmW { uint4 hd, c[2]; };
 
 __device__ __forceinline__ void qm_w_load(const uint8_t* rp, int b, int kq, QmW& w) {
@@ -239,14 +240,6 @@ __device__ __forceinline__ void qm_w_load(const uint8_t* rp, int b, int kq, QmW&
     w.c[0] = *(const uint4*)(blk + 16 + 16 * kq);
     w.c[1] = *(const uint4*)(blk + 80 + 16 * kq);
 }
-// a couple's pieces -> the lane's 8 bytes of each of its two pairs: one exchange between the wave's halves leaves
-// them at bytes 8 kperm(kq) of the pair, kperm = {0, 2, 1, 3}; x is read in the same order, so the dots are the same
-__device__ __forceinline__ void qm_couple(const uint4 c, uint2& a, uint2& b) {
-    const auto x = __builtin_amdgcn_permlane32_swap(c.x, c.z, false, false), y = __builtin_amdgcn_permlane32_swap(c.y, c.w, false, false);
-    a = make_uint2(x[0], y[0]);
-    b = make_uint2(x[1], y[1]);
-}
-__device__ __forceinline__ int qm_kperm(int kq) { return ((kq & 1) << 1) | (kq >> 1); }
 
 // one pass: tokens [c0, c0 + ncl) of the tile, ncl <= 16 CB, against the lane's RG weight rows (row
 // groups of 16: the x fragment of a sub-block feeds RG MFMAs)
@@ -290,8 +283,8 @@ __device__ __forceinline__ void qm_pass(const QmArgs& a, const qmm_moe_tile& tl,
             const Q4kScaleBytes sbt = q4k_scale_bytes(w[g].hd.y, w[g].hd.z, w[g].hd.w);
             scb[g] = ((uint64_t)sbt.sc_hi << 32) | sbt.sc_lo;
             mnb[g] = ((uint64_t)sbt.m_hi << 32) | sbt.m_lo;
-            qm_couple(w[g].c[0], q0[g], q1[g]);
-            qm_couple(w[g].c[1], q2[g], q3[g]);
+            couple_split(w[g].c[0], q0[g], q1[g]);
+            couple_split(w[g].c[1], q2[g], q3[g]);
         }
         // a loop, not unrolled: one qs pair (two sub-blocks) per iteration keeps the register count low
 #pragma unroll 1
@@ -309,7 +302,7 @@ __device__ __forceinline__ void qm_pass(const QmArgs& a, const qmm_moe_tile& tl,
                 }
 #pragma unroll
                 for (int cb = 0; cb < CB; ++cb) {
-                    const uint2 xv = L.x[cur][sb][qm_kperm(kq)][kQmTok * cb + tok];
+                    const uint2 xv = L.x[cur][sb][kperm(kq)][kQmTok * cb + tok];
                     const long xa = (long)(((uint64_t)xv.y << 32) | (uint64_t)xv.x);
                     const float4 s01 = *(const float4*)&L.sd[cur][sb][kQmTok * cb + 4 * kq];
                     const float4 s23 = *(const float4*)&L.sd[cur][sb][kQmTok * cb + 4 * kq + 2];

@@ -57,8 +57,6 @@ struct MBlk {
     uint4 x[4];        // x of the lane's token slot, bytes 64j + 16h..+15 of the block (pair j)
 };
 
-__device__ __forceinline__ int kperm(int h) { return ((h & 1) << 1) | (h >> 1); }
-
 typedef unsigned u32x4v __attribute__((ext_vector_type(4)));
 
 // x through a buffer resource over the call's x: lanes of empty token slots use an offset past its
@@ -79,14 +77,6 @@ __device__ __forceinline__ void mblk_load(MBlk& B, const uint8_t* rp, __amdgpu_b
 #pragma unroll
         for (int j = 0; j < 4; ++j) B.x[j] = xload(rx, xo + (uint32_t)(b * 256 + 64 * j));
     }
-}
-
-// {lane's 8 bytes of pair 2c, lane's 8 bytes of pair 2c+1} from the couple's 16-byte piece
-__device__ __forceinline__ void couple_split(const uint4 v, uint2& p0, uint2& p1) {
-    const auto sx = __builtin_amdgcn_permlane32_swap(v.x, v.z, false, false);
-    const auto sy = __builtin_amdgcn_permlane32_swap(v.y, v.w, false, false);
-    p0 = make_uint2(sx[0], sy[0]);
-    p1 = make_uint2(sx[1], sy[1]);
 }
 
 // adds block b's pair values to acc; a block past the row's end (live = false, b clamped by the

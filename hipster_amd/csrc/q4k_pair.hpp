@@ -260,4 +260,17 @@ __device__ __forceinline__ void stage_xq8_pairs(uint8_t* lds, const int8_t* __re
     __syncthreads();
 }
 
+// The quants of a block on the int8 matrix cores (16 rows a wave, four lanes h = lane / 16 of a row): lane h loads 16-byte
+// piece h of each couple of qs pairs (64 bytes; as four 8-byte pieces, one a pair, the address units set the time).  One
+// exchange between the wave's halves leaves it 8 bytes of each pair, at bytes 8 kperm(h), kperm = {0, 2, 1, 3}; x
+// is read in the same order, so the dots are the same.
+__device__ __forceinline__ int kperm(int h) { return ((h & 1) << 1) | (h >> 1); }
+// {lane's 8 bytes of pair 2c, lane's 8 bytes of pair 2c+1} from the couple's 16-byte piece
+__device__ __forceinline__ void couple_split(const uint4 v, uint2& p0, uint2& p1) {
+    const auto sx = __builtin_amdgcn_permlane32_swap(v.x, v.z, false, false);
+    const auto sy = __builtin_amdgcn_permlane32_swap(v.y, v.w, false, false);
+    p0 = make_uint2(sx[0], sy[0]);
+    p1 = make_uint2(sx[1], sy[1]);
+}
+
 }  // namespace qmm
