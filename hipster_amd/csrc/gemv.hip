@@ -984,14 +984,16 @@ __global__ void __launch_bounds__(kF32mBlock) k_gemv_q4k_f32m(const uint8_t* __r
         // All tasks side by side, 4 k at a time: a task's two chains wait for each of their matrix instructions, the
         // 2 NITER chains of the row hide that and the LDS reads (x of the next 4 k is read ahead).  The next group's
         // weights are loaded into the registers that this one is done with.
+        // (six iterations, K > 5120: x without the read-ahead, whose 48 registers spilled: 17408 x 6144 at four columns 50 -> 31 us)
+        constexpr bool kAhead = NITER < 6;
         f32x4m sa[NITER], sb[NITER];
-        float4 xa[2][NITER], xb[2][NITER];
+        float4 xa[1 + kAhead][NITER], xb[1 + kAhead][NITER];
         auto xread = [&](int q) {
 #pragma unroll
             for (int i = 0; i < NITER; ++i) {
                 const uint8_t* xp = xc + (size_t)min(t + 16 * i, ntask - 1) * 16;
-                xa[q & 1][i] = *(const float4*)(xp + (size_t)(q * kp) * 16);
-                xb[q & 1][i] = *(const float4*)(xp + (size_t)((8 + q) * kp) * 16);
+                xa[kAhead & q][i] = *(const float4*)(xp + (size_t)(q * kp) * 16);
+                xb[kAhead & q][i] = *(const float4*)(xp + (size_t)((8 + q) * kp) * 16);
             }
         };
         auto wread = [&](int part) {
@@ -1005,9 +1007,10 @@ __global__ void __launch_bounds__(kF32mBlock) k_gemv_q4k_f32m(const uint8_t* __r
         };
 #pragma unroll
         for (int i = 0; i < NITER; ++i) sa[i] = sb[i] = f32x4m{0.f, 0.f, 0.f, 0.f};
-        xread(0);
+        if (kAhead) xread(0);
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
+            if (!kAhead) xread(q);
             uint32_t lo[NITER], hi[NITER];
 #pragma unroll
             for (int i = 0; i < NITER; ++i) {
@@ -1016,7 +1019,7 @@ __global__ void __launch_bounds__(kF32mBlock) k_gemv_q4k_f32m(const uint8_t* __r
                 lo[i] = opaque(w & 0x0f0f0f0fu);
                 hi[i] = opaque(w & 0xf0f0f0f0u);
             }
-            if (q < 7) xread(q + 1);
+            if (kAhead && q < 7) xread(q + 1);
             if (q == 3) wread(0);
             if (q == 7) wread(1);
             __builtin_amdgcn_sched_barrier(0);
@@ -1024,8 +1027,8 @@ __global__ void __launch_bounds__(kF32mBlock) k_gemv_q4k_f32m(const uint8_t* __r
             for (int b = 0; b < 4; ++b) {
 #pragma unroll
                 for (int i = 0; i < NITER; ++i) {
-                    sa[i] = __builtin_amdgcn_mfma_f32_4x4x1f32(((const float*)&xa[q & 1][i])[b], (float)((lo[i] >> (8 * b)) & 0xffu), sa[i], 0, 0, 0);
-                    sb[i] = __builtin_amdgcn_mfma_f32_4x4x1f32(((const float*)&xb[q & 1][i])[b], (float)((hi[i] >> (8 * b)) & 0xffu), sb[i], 0, 0, 0);
+                    sa[i] = __builtin_amdgcn_mfma_f32_4x4x1f32(((const float*)&xa[kAhead & q][i])[b], (float)((lo[i] >> (8 * b)) & 0xffu), sa[i], 0, 0, 0);
+                    sb[i] = __builtin_amdgcn_mfma_f32_4x4x1f32(((const float*)&xb[kAhead & q][i])[b], (float)((hi[i] >> (8 * b)) & 0xffu), sb[i], 0, 0, 0);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -1296,12 +1299,13 @@ int qmm_gemv_q4_K_f32(const void* W, const float* x, float* y, int N, int K, int
     if (K <= 6144 && g >= 1) {
         // Four columns at a time on the f32 matrix cores, the rest on the VALU kernel (the same bits).  Measured at
         // 17408 x 5120, M = 4 / 6 / 8: 49 / 69 / 88 us -> 28 / 50 / 53; 1000 x 1536: M = 4 8.9 -> 5.8; 3001 x 6144: 19.7 ->
-        // 17.9.  A remainder of three takes the matrix cores where the VALU kernel is the slower one (26.8 against 36
-        // us at 17408 x 5120, 13.8 against 14.6 at 5120 x 5120; 12.6 against 12.3 at 17408 x 2048, 17.1 against 16.4 at
-        // 3001 x 6144); one or two columns cost the matrix cores as much as four.
+        // 12.6.  A remainder of three takes the matrix cores from K > 3072 on, where three columns of x leave the VALU kernel three
+        // and fewer workgroups a CU (VALU / matrix cores at 1000, 5120 and 17408 rows: K = 3072 7.1 / 7.3, 8.4 / 8.5, 16.9 /
+        // 16.8; K = 3584 8.6 / 8.1, 10.7 / 10.0, 21.5 / 19.4; K = 6144 15.0 / 12.4, 19.4 / 15.4, 43.9 / 29.9); one or two
+        // columns cost the matrix cores as much as four.
         for (int c0 = 0; c0 < ncol;) {
             const int left = ncol - c0;
-            const bool mfma = left >= 4 || (left == 3 && K > 2048 && K <= 5120);
+            const bool mfma = left >= 4 || (left == 3 && K > 3072);
             const int nc = mfma ? min(4, left) : min(g, left);
             const float* xc = x + (size_t)c0 * K;
             float* yc = y + (size_t)c0 * N;
