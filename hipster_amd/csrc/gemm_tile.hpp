@@ -24,13 +24,14 @@
 //   300 x 17408 x 5120     136 -> 67    231 -> 91    197 -> 76    169 -> 97
 //   300 x 5120 x 17408     416 -> 109   758 -> 118   635 -> 108   527 -> 101
 //   40 x 1024 x 5120       118 -> 9     202 -> 15    162 -> 10    136 -> 8
-// What bounds it.  With many rows the matrix cores at the clock that the card's power leaves them.  With few rows the vector
-// memory path: a load of one row per lane keeps the address units busy about as long whatever its width, and without the
-// weight loads 300 x 17408 x 5120 took 53 us instead of 73 (no dequantisation 62, no matrix instructions 59, eight
-// stages instead of four the same).  Hence the scales and high bits of four steps in one load (a step's loads
-// Q4_K 2 -> 1.25, Q5_K 3 -> 1.5, Q6_K 4 -> 2, Q5_1 4 -> 2) and the loads of a step spread over its slices.  Measured and
-// not kept: the weight rows through LDS by DMA with consecutive lanes on consecutive bytes (the same times: the LDS
-// traffic and the waits took back what the address units gained), six and eight stages.
+// What bounds it (counters).  With many rows the card's power: 2048 x 17408 x 5120 Q4_K keeps the matrix cores busy 67% of the
+// time at 1.57 GHz.  With few rows the vector memory path: the address units are busy 47% (300 x 17408 x 5120) to 76% (300 x
+// 5120 x 17408 Q6_K, k_gemm_few) of the time at 34 cycles an instruction, since a load of one row per lane keeps them about as
+// long whatever its width; without the weight loads the first took 53 us instead of 73 (no dequantisation 62, no
+// matrix instructions 59, eight stages instead of four the same).  Hence the scales and high bits of four steps in one
+// load (a step's loads Q4_K 2 -> 1.25, Q5_K 3 -> 1.5, Q6_K 4 -> 2, Q5_1 4 -> 2) and the loads of a step spread over its
+// slices.  Measured and not kept: the weight rows through LDS by DMA with consecutive lanes on consecutive bytes (the same
+// times: the LDS traffic and the waits took back what the address units gained), six and eight stages.
 #pragma once
 #include <type_traits>
 
