@@ -19,11 +19,11 @@
 // Measured against the 256 x 256 kernel it replaced, which dequantised through LDS and whose flat-form DMA made
 // the compiler wait for every load in flight twice a step (calls in a stream, weights rotated, us):
 //   M x N x K              Q4_K         Q6_K         Q8_0         bf16
-//   2048 x 17408 x 5120    392 -> 319   663 -> 369   602 -> 336   500 -> 355
-//   2048 x 5120 x 17408    473 -> 310   712 -> 369   636 -> 333   547 -> 364
-//   300 x 17408 x 5120     136 -> 67    231 -> 91    197 -> 76    169 -> 97
-//   300 x 5120 x 17408     416 -> 109   758 -> 118   635 -> 108   527 -> 101
-//   40 x 1024 x 5120       118 -> 9     202 -> 15    162 -> 10    136 -> 8
+//   2048 x 17408 x 5120    383 -> 327   681 -> 369   585 -> 347   503 -> 374
+//   2048 x 5120 x 17408    485 -> 322   752 -> 387   659 -> 354   566 -> 390
+//   300 x 17408 x 5120     135 -> 68    234 -> 89    201 -> 77    168 -> 97
+//   300 x 5120 x 17408     415 -> 116   729 -> 122   641 -> 112   528 -> 108
+//   40 x 1024 x 5120       119 -> 9     202 -> 14    162 -> 10    136 -> 9
 // What bounds it (counters).  With many rows the card's power: 2048 x 17408 x 5120 Q4_K keeps the matrix cores busy 67% of the
 // time at 1.57 GHz.  With few rows the vector memory path: the address units are busy 47% (300 x 17408 x 5120) to 76% (300 x
 // 5120 x 17408 Q6_K, k_gemm_few) of the time at 34 cycles an instruction, since a load of one row per lane keeps them about as
